@@ -86,9 +86,9 @@ __device__ __forceinline__ uint32_t fta_range_bits(int lo, int hi) {
 
 // Column masks of the WG's query tiles for KV blocks [seg0, seg0 + segn), then
 // the ascending union list.  Returns the list length.
-template <int T>
+template <int T, typename LT>
 __device__ int fta_build_q_masks(const AttnArgs& a, int bh, int p0, int seg0, int segn, uint32_t (*sMask)[kSeg],
-                                 int* sList, int* s_tmp) {
+                                 LT* sList, int* s_tmp) {
     const int tid = threadIdx.x;
     for (int i = tid; i < T * kSeg; i += blockDim.x) sMask[i / kSeg][i % kSeg] = 0u;
     __syncthreads();
@@ -139,7 +139,7 @@ __device__ int fta_build_q_masks(const AttnArgs& a, int bh, int p0, int seg0, in
             if (w < wave) wbase += t;
             tot += t;
         }
-        if (any) sList[U + wbase + x - any] = ml;
+        if (any) sList[U + wbase + x - any] = (LT)ml;
         __syncthreads();
         U += tot;
     }
@@ -379,6 +379,17 @@ __global__ __launch_bounds__(NW * 64, 1) void fta_sparse_fwd_kernel(AttnArgs a) 
 // the swizzled row layout, NST - 1 chunks ahead of the MFMAs, so the gather
 // latency is hidden behind the work of the chunks in flight and no registers
 // stage the copies.
+//
+// What bounds it: at D = 128 the matrix pipe and the power-limited clock (44% MFMA
+// busy, 0.98 PFLOP/s on dense lists, 80% of a large library GEMM on the same card);
+// at D = 64 instruction issue (per 64 x 32 scores 169 VALU instructions against 16
+// MFMAs).  At D = 64 two waves per SIMD left both pipes idle a third of the time,
+// so the kernel is held to 128 registers and three stages and two workgroups
+// share a CU.  Operand fragments are read a fixed few MFMAs ahead (PDK, PDV) behind
+// scheduling fences: left alone the compiler either keeps a whole chunk's fragments
+// in registers (156 at D = 64) or waits out one LDS latency per MFMA.  B2 N8192 H16
+// D64 fp16, lists of every block: 0.80 -> 0.66 ms; one list of 16 blocks per query:
+// 0.74 -> 0.61 ms (whole call); B1 N16384 H16 D128 dense lists: 1.95 -> 1.88 ms.
 // ----------------------------------------------------------------------------
 template <int D, int NW>
 struct FwdPipeShape {
@@ -387,37 +398,120 @@ struct FwdPipeShape {
     static constexpr int LQ = SLOTS / (64 * NW);    // DMA instructions per wave per tensor
     static constexpr int TEN_B = SLOTS * 16;        // bytes per tensor chunk
     static constexpr int STAGE_B = 2 * TEN_B;       // K then V
-    static constexpr int NST = (3 * STAGE_B <= 96 * 1024 && D <= 64) ? 4 : 3;
+    static constexpr int NST = 3;                   // stage buffers (at D = 64 two WGs share a CU)
     static_assert(SLOTS % (64 * NW) == 0, "whole DMA instructions per wave");
     static_assert(NST * STAGE_B + NW * kSeg * 4 + kSeg * 4 <= 150 * 1024, "LDS budget");
 };
 
-// Empty asm with every fragment as a read-write VGPR operand: all loads into
-// `f` complete before it, and none can be moved below it.
-typedef unsigned int fta_u32x4v __attribute__((ext_vector_type(4)));
-template <int KS>
-__device__ __forceinline__ void fta_pin_frags(uint4 (&f)[2][KS]) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int k = 0; k < KS; k += 4) {
-            fta_u32x4v x0 = __builtin_bit_cast(fta_u32x4v, f[h][k]);
-            fta_u32x4v x1 = __builtin_bit_cast(fta_u32x4v, f[h][(k + 1) % KS]);
-            fta_u32x4v x2 = __builtin_bit_cast(fta_u32x4v, f[h][(k + 2) % KS]);
-            fta_u32x4v x3 = __builtin_bit_cast(fta_u32x4v, f[h][(k + 3) % KS]);
-            asm volatile("" : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(x3));
-            f[h][k] = __builtin_bit_cast(uint4, x0);
-            if (k + 1 < KS) f[h][k + 1] = __builtin_bit_cast(uint4, x1);
-            if (k + 2 < KS) f[h][k + 2] = __builtin_bit_cast(uint4, x2);
-            if (k + 3 < KS) f[h][k + 3] = __builtin_bit_cast(uint4, x3);
+// The walk of a pipelined forward / dQ workgroup over its part of a segment's
+// union list: 64-key chunks, `nch` per listed block.  The list entry and the
+// tile mask of the block after the current one are read from LDS one chunk
+// ahead, so no LDS round trip sits between a chunk's barrier and its first
+// MFMA (reading them in place cost two dependent LDS reads per chunk in every
+// wave at once).  A wave's mask row is first compacted to list order.
+struct QWalk {
+    const uint16_t* list;  // block (relative to the segment) at each list position of the part
+    const uint32_t* mask;  // this wave's column mask at each list position of the part
+    int n, nch;            // list positions of the part, chunks per block
+    int iu, ich, im;       // next chunk to gather: list position, chunk of the block, block
+    int cu, cch, cm;       // current chunk: list position, chunk of the block, block
+    uint32_t cmk;          // mask of the current block
+    int v_im, v_cm;        // read ahead: blocks at iu + 1 and cu + 1, mask at cu + 1
+    uint32_t v_cmk;
+
+    __device__ __forceinline__ void start(const uint16_t* l, const uint32_t* m, int n_, int nch_) {
+        list = l;
+        mask = m;
+        n = n_;
+        nch = nch_;
+        iu = ich = cu = cch = 0;
+        im = cm = __builtin_amdgcn_readfirstlane((int)list[0]);
+        cmk = __builtin_amdgcn_readfirstlane(mask[0]);
+        v_im = v_cm = list[min(1, n - 1)];
+        v_cmk = mask[min(1, n - 1)];
+    }
+    __device__ __forceinline__ void next_gather() {
+        if (++ich == nch) {
+            ich = 0;
+            ++iu;
+            im = __builtin_amdgcn_readfirstlane(v_im);
+            v_im = list[min(iu + 1, n - 1)];
         }
+    }
+    __device__ __forceinline__ void next_chunk() {
+        if (++cch == nch) {
+            cch = 0;
+            ++cu;
+            cm = __builtin_amdgcn_readfirstlane(v_cm);
+            cmk = __builtin_amdgcn_readfirstlane(v_cmk);
+        }
+    }
+    // reads ahead for the next next_chunk (issued early in a chunk)
+    __device__ __forceinline__ void read_ahead() {
+        const int p = min(cu + 1, n - 1);
+        v_cm = list[p];
+        v_cmk = mask[p];
+    }
+};
+
+// Reorders a wave's mask row from block order to list order in place (list
+// entries ascend, so entry u reads at or after position u; a wave's LDS
+// accesses stay in order).
+__device__ __forceinline__ void fta_compact_masks(uint32_t* row, const uint16_t* list, int U) {
+    const int lane = threadIdx.x & 63;
+    for (int u0 = 0; u0 < U; u0 += 64) {
+        const int u = u0 + lane;
+        const uint32_t m = (u < U) ? row[list[u]] : 0u;
+        if (u < U) row[u] = m;
+    }
+}
+
+// Gathers the 64 K and V rows at padded key offset kb (the chunk's first row,
+// relative to the sequence) into the stage at LDS address sb: one SGPR base per
+// tensor and a 32-bit byte offset per lane.  Rows outside [0, N) are clamped
+// into it (masked by the caller).
+template <int D, int NW>
+__device__ __forceinline__ void fta_gather_kv(const AttnArgs& a, const uint16_t* kp, const uint16_t* vp, int kb,
+                                              bool inside, const uint32_t* koff, const uint32_t* voff, uint32_t sb,
+                                              int wave, int lane) {
+    using Sh = FwdPipeShape<D, NW>;
+    using SW = FtaSwz<Sh::QSEG>;
+    const int t0 = min(max(kb, 0), a.N - 1);
+    const uint16_t* kbp = kp + (int64_t)t0 * a.k_sn;
+    const uint16_t* vbp = vp + (int64_t)t0 * a.v_sn;
+    if (inside) {
+#pragma unroll
+        for (int i = 0; i < Sh::LQ; ++i) fta_dma16_so(kbp, koff[i], sb + (i * NW + wave) * 1024);
+#pragma unroll
+        for (int i = 0; i < Sh::LQ; ++i) fta_dma16_so(vbp, voff[i], sb + Sh::TEN_B + (i * NW + wave) * 1024);
+    } else {
+#pragma unroll
+        for (int i = 0; i < Sh::LQ; ++i) {
+            const int sidx = (i * NW + wave) * 64 + lane;
+            const int row = sidx / Sh::QSEG;
+            int j = SW::slot(row, sidx - row * Sh::QSEG);
+            if (j * 8 >= a.Dreal) j = 0;
+            const uint32_t rel = (uint32_t)(min(max(kb + row, 0), a.N - 1) - t0);  // 0 .. 63
+            fta_dma16_so(kbp, 2u * (rel * (uint32_t)a.k_sn + j * 8), sb + (i * NW + wave) * 1024);
+            fta_dma16_so(vbp, 2u * (rel * (uint32_t)a.v_sn + j * 8), sb + Sh::TEN_B + (i * NW + wave) * 1024);
+        }
+    }
+}
+
+// f(integral_constant<int, I>) for I = I0 .. N - 1
+template <int I, int N, typename F>
+__device__ __forceinline__ void fta_for(F& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        fta_for<I + 1, N>(f);
+    }
 }
 
 // SPLIT: workgroup (tiles, part sp) walks union positions [sp U / nsplit,
 // (sp + 1) U / nsplit) of each mask segment and writes its unnormalised partial
 // output, running max and sum instead of o and lse.
 template <int DT, int D, int NW, bool SPLIT>
-__global__ __launch_bounds__(NW * 64, 1) void fta_sparse_fwd_pipe_kernel(AttnArgs a) {
+__global__ __launch_bounds__(NW * 64, D <= 64 ? 4 : 1) void fta_sparse_fwd_pipe_kernel(AttnArgs a) {
     using E = Elem<DT>;
     using Sh = FwdPipeShape<D, NW>;
     constexpr int QSEG = Sh::QSEG, LQ = Sh::LQ, NST = Sh::NST;
@@ -427,7 +521,7 @@ __global__ __launch_bounds__(NW * 64, 1) void fta_sparse_fwd_pipe_kernel(AttnArg
     constexpr int DT32 = D / 32;
     __shared__ __align__(1024) unsigned char sStage[NST][Sh::STAGE_B];
     __shared__ uint32_t sMask[T][kSeg];
-    __shared__ int sList[kSeg];
+    __shared__ uint16_t sList[kSeg];
     __shared__ int s_tmp[8];
 
     const int wgi = fta_xcd_remap(blockIdx.x, a.total);
@@ -474,18 +568,25 @@ __global__ __launch_bounds__(NW * 64, 1) void fta_sparse_fwd_pipe_kernel(AttnArg
     float m_run = -FTA_INF, l_run = 0.f;
 
     // Per-lane DMA sources: instruction i of this wave fills the 1 KB block
-    // i * NW + wave of each tensor chunk; koff / voff = row * stride + column.
-    int koff[LQ], voff[LQ];
+    // i * NW + wave of each tensor chunk; koff / voff = row * stride + column, in bytes.
+    uint32_t koff[LQ], voff[LQ];
 #pragma unroll
     for (int i = 0; i < LQ; ++i) {
         const int sidx = (i * NW + wave) * 64 + lane;
         const int row = sidx / QSEG;
         int j = SW::slot(row, sidx - row * QSEG);
         if (j * 8 >= a.Dreal) j = 0;  // columns past D: zero q columns / outputs never stored
-        koff[i] = row * (int)a.k_sn + j * 8;
-        voff[i] = row * (int)a.v_sn + j * 8;
+        koff[i] = 2u * (row * (uint32_t)a.k_sn + j * 8);  // at most 63 * 2^24 * 2 + 256 < 2^32
+        voff[i] = 2u * (row * (uint32_t)a.v_sn + j * 8);
     }
     const uint32_t lds0 = fta_lds_addr(&sStage[0][0]);
+    constexpr int PDK = D <= 64 ? 3 : 6, PDV = D <= 64 ? 2 : 4;
+    // per-lane byte offsets of the operand fragments in a stage: K rows, V transposed.
+    // The other k slices / column tiles differ by an XOR of their slot bits (rows are
+    // a multiple of 64 bytes and the tile base of 1 KB, so the swizzle stays inside).
+    const uint32_t kro0 = 2u * SW::off(lane & 31, hf);
+    const int vr = 4 * (lane >> 5) + ((lane & 15) >> 2), vc = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    const uint32_t vro0[2] = {2u * (SW::off(vr, vc >> 3) + (vc & 7)), 2u * (SW::off(vr + 8, vc >> 3) + (vc & 7))};
     const int nch = (a.kvb + 63) >> 6;
 
     for (int seg0 = 0; seg0 < a.Mkv; seg0 += kSeg) {
@@ -500,38 +601,21 @@ __global__ __launch_bounds__(NW * 64, 1) void fta_sparse_fwd_pipe_kernel(AttnArg
         if (u_n == 0) continue;
         const int iters = u_n * nch;
 
-        // gather chunk `it` (64 keys of union block it / nch) into stage buffer st
-        auto issue = [&](int st, int it) {
-            const uint32_t sb = lds0 + st * Sh::STAGE_B;
-            const int u = u_lo + it / nch, ch = it - (it / nch) * nch;
-            const int m = __builtin_amdgcn_readfirstlane(seg0 + sList[u]);
-            const int kb = m * a.kvb - a.kv_pad + ch * 64;
-            const int rem = a.kvb - ch * 64;
-            if (kb >= 0 && kb + 64 <= a.N && rem >= 64) {
-                const uint16_t* kbp = kp + (int64_t)kb * a.k_sn;
-                const uint16_t* vbp = vp + (int64_t)kb * a.v_sn;
-#pragma unroll
-                for (int i = 0; i < LQ; ++i) fta_dma16_at(kbp + koff[i], sb + (i * NW + wave) * 1024);
-#pragma unroll
-                for (int i = 0; i < LQ; ++i) fta_dma16_at(vbp + voff[i], sb + Sh::TEN_B + (i * NW + wave) * 1024);
-            } else {  // chunk at a sequence / block edge: clamp rows into [0, N) (masked below)
-#pragma unroll
-                for (int i = 0; i < LQ; ++i) {
-                    const int sidx = (i * NW + wave) * 64 + lane;
-                    const int row = sidx / QSEG;
-                    int j = SW::slot(row, sidx - row * QSEG);
-                    if (j * 8 >= a.Dreal) j = 0;
-                    const int t = min(max(kb + row, 0), a.N - 1);
-                    fta_dma16_at(kp + (int64_t)t * a.k_sn + j * 8, sb + (i * NW + wave) * 1024);
-                    fta_dma16_at(vp + (int64_t)t * a.v_sn + j * 8, sb + Sh::TEN_B + (i * NW + wave) * 1024);
-                }
-            }
+        fta_compact_masks(sMask[wave], sList, U);
+        QWalk w;
+        w.start(sList + u_lo, sMask[wave] + u_lo, u_n, nch);
+        // gather the walk's next chunk into stage buffer st
+        auto issue = [&](int st) {
+            const int kb = (seg0 + w.im) * a.kvb - a.kv_pad + w.ich * 64;
+            const bool inside = kb >= 0 && kb + 64 <= a.N && a.kvb - w.ich * 64 >= 64;
+            fta_gather_kv<D, NW>(a, kp, vp, kb, inside, koff, voff, lds0 + st * Sh::STAGE_B, wave, lane);
+            w.next_gather();
         };
 
         fta_wait_vmcnt<0>();  // register loads complete before the DMA stream
 #pragma unroll
         for (int k = 0; k < NST - 1; ++k)
-            if (k < iters) issue(k, k);
+            if (k < iters) issue(k);
         int cur = 0;
         for (int it = 0; it < iters; ++it) {
             // chunk it resident: chunks issued so far = min(iters, it + NST - 1)
@@ -540,37 +624,35 @@ __global__ __launch_bounds__(NW * 64, 1) void fta_sparse_fwd_pipe_kernel(AttnArg
             else
                 fta_wait_vmcnt<0>();
             __syncthreads();  // chunk it visible; every wave is past chunk it - 1
-            if (it + NST - 1 < iters) issue(cur == 0 ? NST - 1 : cur - 1, it + NST - 1);
-
-            const int u = u_lo + it / nch, ch = it - (it / nch) * nch;
-            const int ml = sList[u];
-            const int m = seg0 + ml;
-            const int kb = m * a.kvb - a.kv_pad + ch * 64;
-            const int rem = a.kvb - ch * 64;
-            const uint32_t mk = __builtin_amdgcn_readfirstlane(sMask[wave][ml]);
+            if (it + NST - 1 < iters) issue(cur == 0 ? NST - 1 : cur - 1);
+            w.read_ahead();
+            const int kb = (seg0 + w.cm) * a.kvb - a.kv_pad + w.cch * 64;
+            const int rem = a.kvb - w.cch * 64;
+            const uint32_t mk = w.cmk;
             if (mk) {
-                const uint16_t* kbase = reinterpret_cast<const uint16_t*>(&sStage[cur][0]);
-                const uint16_t* vbase = kbase + Sh::TEN_B / 2;
+                const uint32_t kbase = lds0 + cur * Sh::STAGE_B, vbase = kbase + Sh::TEN_B;
                 f32x16 s[2];
+                {
+                    constexpr int PD = PDK;
+                    uint4 fr[PD + 1];
+                    auto load = [&](auto nn) __attribute__((always_inline)) {
+                        constexpr int n = decltype(nn)::value;
+                        if constexpr (n < 2 * KS)
+                            fr[n % (PD + 1)] = fta_lds_b128(((kbase + kro0) ^ ((n >> 1) * 32)) + (n & 1) * 32 * QSEG * 16);
+                    };
+                    auto slot = [&](auto nn) __attribute__((always_inline)) {
+                        constexpr int n = decltype(nn)::value;
+                        if constexpr (n % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+                        load(std::integral_constant<int, n + PD>{});
+                        if constexpr (n < 2) {
 #pragma unroll
-                for (int sb = 0; sb < 2; ++sb)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) s[sb][i] = 0.f;
-                // all K fragments of the chunk first, then the MFMAs: one LDS
-                // latency per chunk instead of one per MFMA
-                uint4 ka[2][KS];
-#pragma unroll
-                for (int ks = 0; ks < KS; ++ks) {
-                    ka[0][ks] = *reinterpret_cast<const uint4*>(kbase + SW::off(lane & 31, 2 * ks + hf));
-                    ka[1][ks] = *reinterpret_cast<const uint4*>(kbase + SW::off(32 + (lane & 31), 2 * ks + hf));
-                }
-                // the empty asm takes every fragment as an operand, so the loads
-                // cannot sink to their MFMAs (which exposes one LDS latency per MFMA)
-                fta_pin_frags<KS>(ka);
-#pragma unroll
-                for (int ks = 0; ks < KS; ++ks) {
-                    s[0] = E::mma(ka[0][ks], qf[ks], s[0]);
-                    s[1] = E::mma(ka[1][ks], qf[ks], s[1]);
+                            for (int i = 0; i < 16; ++i) s[n][i] = 0.f;
+                        }
+                        s[n & 1] = E::mma(fr[n % (PD + 1)], qf[n >> 1], s[n & 1]);
+                    };
+                    fta_for<0, PD>(load);
+                    fta_for<0, 2 * KS>(slot);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
                 // valid keys of the chunk: [klo, khi) relative to kb (wave-uniform).
                 // Keys outside it get -inf scores in place (chunks at a sequence end
@@ -609,28 +691,39 @@ __global__ __launch_bounds__(NW * 64, 1) void fta_sparse_fwd_pipe_kernel(AttnArg
                 }
                 const float mc = !colok ? FTA_INF : (m_run == -FTA_INF) ? 0.f : m_run * a.c;
                 float ls = 0.f;
-                uint4 pf[4];
+                {
+                    constexpr int PD = PDV, NM = 4 * DT32;
+                    uint4 fr[PD + 1];
+                    uint32_t pw[4];
+                    auto load = [&](auto nn) __attribute__((always_inline)) {
+                        constexpr int n = decltype(nn)::value;
+                        if constexpr (n < NM)
+                            fr[n % (PD + 1)] = fta_lds_tr(((vbase + vro0[0]) ^ ((n % DT32) * 64)) + (n / DT32) * 16 * QSEG * 16,
+                                                          ((vbase + vro0[1]) ^ ((n % DT32) * 64)) + (n / DT32) * 16 * QSEG * 16);
+                    };
+                    auto slot = [&](auto nn) __attribute__((always_inline)) {
+                        constexpr int n = decltype(nn)::value, ks = n / DT32;
+                        if constexpr (n % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+                        load(std::integral_constant<int, n + PD>{});
+                        if constexpr (n % DT32 == 0) {
+                            float pv[8];
 #pragma unroll
-                for (int ks = 0; ks < 4; ++ks) {
-                    float pv[8];
+                            for (int e = 0; e < 8; ++e) {
+                                pv[e] = fta_exp2(fmaf(s[ks >> 1][8 * (ks & 1) + e], a.c, -mc));
+                                ls += pv[e];
+                            }
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        pv[e] = fta_exp2(fmaf(s[ks >> 1][8 * (ks & 1) + e], a.c, -mc));
-                        ls += pv[e];
-                    }
-                    pf[ks] = make_uint4(E::pack2(pv[0], pv[1]), E::pack2(pv[2], pv[3]), E::pack2(pv[4], pv[5]),
-                                        E::pack2(pv[6], pv[7]));
+                            for (int e = 0; e < 4; ++e) pw[e] = E::pack2(pv[2 * e], pv[2 * e + 1]);
+                        }
+                        oacc[n % DT32] = E::mma(fr[n % (PD + 1)], make_uint4(pw[0], pw[1], pw[2], pw[3]), oacc[n % DT32]);
+                    };
+                    fta_for<0, PD>(load);
+                    fta_for<0, NM>(slot);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
                 l_run += ls;
-#pragma unroll
-                for (int ks = 0; ks < 4; ++ks) {
-#pragma unroll
-                    for (int dt = 0; dt < DT32; ++dt) {
-                        const uint4 vf = fta_tr_frag_sw<QSEG>(vbase, ks * 16, dt * 32, lane);
-                        oacc[dt] = E::mma(vf, pf[ks], oacc[dt]);
-                    }
-                }
             }
+            w.next_chunk();
             cur = (cur == NST - 1) ? 0 : cur + 1;
         }
         __syncthreads();  // every wave is done with sMask / sList before the next segment rebuilds them
@@ -953,7 +1046,7 @@ __global__ __launch_bounds__(512, 1) void fta_sparse_dq_pipe_kernel(AttnArgs a) 
     constexpr int DT32 = D / 32;
     __shared__ __align__(1024) unsigned char sStage[NST][Sh::STAGE_B];
     __shared__ uint32_t sMask[T][kSeg];
-    __shared__ int sList[kSeg];
+    __shared__ uint16_t sList[kSeg];
     __shared__ int s_tmp[8];
 
     const int wgi = fta_xcd_remap(blockIdx.x, a.total);
@@ -1006,16 +1099,16 @@ __global__ __launch_bounds__(512, 1) void fta_sparse_dq_pipe_kernel(AttnArgs a) 
         for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
 
     // Per-lane DMA sources: instruction i of this wave fills the 1 KB block
-    // i * NW + wave of each tensor chunk; koff / voff = row * stride + column.
-    int koff[LQ], voff[LQ];
+    // i * NW + wave of each tensor chunk; koff / voff = row * stride + column, in bytes.
+    uint32_t koff[LQ], voff[LQ];
 #pragma unroll
     for (int i = 0; i < LQ; ++i) {
         const int sidx = (i * NW + wave) * 64 + lane;
         const int row = sidx / QSEG;
         int j = SW::slot(row, sidx - row * QSEG);
-        if (j * 8 >= a.Dreal) j = 0;  // columns past D: zero q / dO columns, outputs never stored
-        koff[i] = row * (int)a.k_sn + j * 8;
-        voff[i] = row * (int)a.v_sn + j * 8;
+        if (j * 8 >= a.Dreal) j = 0;  // columns past D: zero q columns / outputs never stored
+        koff[i] = 2u * (row * (uint32_t)a.k_sn + j * 8);  // at most 63 * 2^24 * 2 + 256 < 2^32
+        voff[i] = 2u * (row * (uint32_t)a.v_sn + j * 8);
     }
     const uint32_t lds0 = fta_lds_addr(&sStage[0][0]);
     const int nch = (a.kvb + 63) >> 6;
@@ -1032,53 +1125,35 @@ __global__ __launch_bounds__(512, 1) void fta_sparse_dq_pipe_kernel(AttnArgs a) 
         if (u_n == 0) continue;
         const int iters = u_n * nch;
 
-        auto issue = [&](int st, int it) {
-            const uint32_t sb = lds0 + st * Sh::STAGE_B;
-            const int u = u_lo + it / nch, ch = it - (it / nch) * nch;
-            const int m = __builtin_amdgcn_readfirstlane(seg0 + sList[u]);
-            const int kb = m * a.kvb - a.kv_pad + ch * 64;
-            const int rem = a.kvb - ch * 64;
-            if (kb >= 0 && kb + 64 <= a.N && rem >= 64) {
-                const uint16_t* kbp = kp + (int64_t)kb * a.k_sn;
-                const uint16_t* vbp = vp + (int64_t)kb * a.v_sn;
-#pragma unroll
-                for (int i = 0; i < LQ; ++i) fta_dma16_at(kbp + koff[i], sb + (i * NW + wave) * 1024);
-#pragma unroll
-                for (int i = 0; i < LQ; ++i) fta_dma16_at(vbp + voff[i], sb + Sh::TEN_B + (i * NW + wave) * 1024);
-            } else {  // chunk at a sequence / block edge: clamp rows into [0, N) (masked below)
-#pragma unroll
-                for (int i = 0; i < LQ; ++i) {
-                    const int sidx = (i * NW + wave) * 64 + lane;
-                    const int row = sidx / QSEG;
-                    int j = SW::slot(row, sidx - row * QSEG);
-                    if (j * 8 >= a.Dreal) j = 0;
-                    const int t = min(max(kb + row, 0), a.N - 1);
-                    fta_dma16_at(kp + (int64_t)t * a.k_sn + j * 8, sb + (i * NW + wave) * 1024);
-                    fta_dma16_at(vp + (int64_t)t * a.v_sn + j * 8, sb + Sh::TEN_B + (i * NW + wave) * 1024);
-                }
-            }
+        fta_compact_masks(sMask[wave], sList, U);
+        QWalk w;
+        w.start(sList + u_lo, sMask[wave] + u_lo, u_n, nch);
+        // gather the walk's next chunk into stage buffer st
+        auto issue = [&](int st) {
+            const int kb = (seg0 + w.im) * a.kvb - a.kv_pad + w.ich * 64;
+            const bool inside = kb >= 0 && kb + 64 <= a.N && a.kvb - w.ich * 64 >= 64;
+            fta_gather_kv<D, NW>(a, kp, vp, kb, inside, koff, voff, lds0 + st * Sh::STAGE_B, wave, lane);
+            w.next_gather();
         };
 
         fta_wait_vmcnt<0>();  // register loads complete before the DMA stream
 #pragma unroll
         for (int k = 0; k < NST - 1; ++k)
-            if (k < iters) issue(k, k);
+            if (k < iters) issue(k);
         int cur = 0;
         for (int it = 0; it < iters; ++it) {
+            // chunk it resident: chunks issued so far = min(iters, it + NST - 1)
             if (it + NST - 2 < iters)
                 fta_wait_vmcnt<2 * LQ * (NST - 2)>();
             else
                 fta_wait_vmcnt<0>();
             __syncthreads();  // chunk it visible; every wave is past chunk it - 1
-            if (it + NST - 1 < iters) issue(cur == 0 ? NST - 1 : cur - 1, it + NST - 1);
-
-            const int u = u_lo + it / nch, ch = it - (it / nch) * nch;
-            const int ml = sList[u];
-            const int m = seg0 + ml;
-            const int kb = m * a.kvb - a.kv_pad + ch * 64;
-            const int rem = a.kvb - ch * 64;
+            if (it + NST - 1 < iters) issue(cur == 0 ? NST - 1 : cur - 1);
+            w.read_ahead();
+            const int kb = (seg0 + w.cm) * a.kvb - a.kv_pad + w.cch * 64;
+            const int rem = a.kvb - w.cch * 64;
             const bool two = rem > 32;
-            const uint32_t mk = __builtin_amdgcn_readfirstlane(sMask[wave][ml]);
+            const uint32_t mk = w.cmk;
             if (mk) {
                 const uint16_t* kbase = reinterpret_cast<const uint16_t*>(&sStage[cur][0]);
                 const uint16_t* vbase = kbase + Sh::TEN_B / 2;
@@ -1148,6 +1223,7 @@ __global__ __launch_bounds__(512, 1) void fta_sparse_dq_pipe_kernel(AttnArgs a) 
                         acc[dt] = E::mma(fta_tr_frag_sw<QSEG>(kbase, ks * 16, dt * 32, lane), dsf[ks], acc[dt]);
                 }
             }
+            w.next_chunk();
             cur = (cur == NST - 1) ? 0 : cur + 1;
         }
         __syncthreads();  // every wave is done with sMask / sList before the next segment rebuilds them
@@ -2081,10 +2157,14 @@ void fill_common(AttnArgs& a, int H, int N, int D, int g, int kvb, int qph, int 
     a.c = scale * 1.4426950408889634f;
 }
 
+// Token strides whose byte offsets over a 64-row tile fit the 32-bit lane offsets of
+// the gathers (64 * 2^24 * 2 bytes = 2^31); others run on the register-staged kernels.
+bool narrow_stride(int64_t sn) { return sn >= 0 && sn <= (1 << 24); }
+
 template <int DT>
 int launch_fwd_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
     // the pipelined kernel keeps per-lane row offsets (64 rows x stride) in 32 bits
-    const bool pipe_ok = a.k_sn <= (1 << 24) && a.v_sn <= (1 << 24);
+    const bool pipe_ok = narrow_stride(a.k_sn) && narrow_stride(a.v_sn);
     switch (Dk) {
 #define FTA_FWD(DK, TPW, NW)                                                                              \
     case DK:                                                                                              \
@@ -2128,7 +2208,7 @@ int launch_fwd_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
 template <int DT>
 int launch_dq_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
     // the pipelined kernel keeps per-lane row offsets (64 rows x stride) in 32 bits
-    const bool pipe_ok = a.k_sn <= (1 << 24) && a.v_sn <= (1 << 24);
+    const bool pipe_ok = narrow_stride(a.k_sn) && narrow_stride(a.v_sn);
     // split walks (decided by the caller, grid included): the pipelined kernels (D 64 /
     // 128) or the register-staged ones (D 160 / 256)
     const bool split = a.nsplit > 1;
@@ -2408,8 +2488,8 @@ int fta_sparse_attn_fwd_gqa(const void* q, const int64_t* q_strides, const void*
     // split walks (small grids, pipelined kernel, workspace for the parts)
     const int ns = fwd_nsplit(B, H, G);
     const bool split = ns > 1 && workspace != nullptr &&
-                       workspace_bytes >= fwd_bytes(B, H) + split_bytes(B, H, G, ns) && k_strides[2] <= (1 << 24) &&
-                       v_strides[2] <= (1 << 24);
+                       workspace_bytes >= fwd_bytes(B, H) + split_bytes(B, H, G, ns) && narrow_stride(k_strides[2]) &&
+                       narrow_stride(v_strides[2]);
     a.nsplit = split ? ns : 1;
     a.nbh = B * H;
     a.npq = G.Npq;
@@ -2528,7 +2608,7 @@ int bwd_dq_impl(const int32_t* head_perm, const void* q, const int64_t* q_stride
     a.wg_per_bh = (G.Npq + 32 * Tq - 1) / (32 * Tq);
     // small grids: each workgroup's union walk in 2-4 parts, summed by fta_dq_combine_kernel
     const int ns = dq_nsplit(B, H, G);
-    const bool pipe_ok = a.k_sn <= (1 << 24) && a.v_sn <= (1 << 24);
+    const bool pipe_ok = narrow_stride(a.k_sn) && narrow_stride(a.v_sn);
     const bool split = ns > 1 && (G.Dk > 128 || pipe_ok) && split_ws != nullptr &&
                        split_avail >= dq_split_bytes(B, H, G, ns);
     a.nsplit = split ? ns : 1;

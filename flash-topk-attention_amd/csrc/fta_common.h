@@ -180,6 +180,21 @@ __device__ __forceinline__ uint4 fta_tr_frag_sw(const uint16_t* tile, int k0, in
     return make_uint4(l2.x, l2.y, h2.x, h2.y);
 }
 
+// LDS reads by byte address (fta_lds_addr + offset): 16 bytes, and the two halves
+// of a transposed fragment (fta_tr_frag_sw) whose addresses the caller holds.
+// x(r) repeats every 16 rows, so a fragment 16 rows down is at a constant offset.
+__device__ __forceinline__ uint4 fta_lds_b128(uint32_t addr) {
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) const u32x4 lds_u32x4;
+    return __builtin_bit_cast(uint4, *(lds_u32x4*)addr);
+}
+__device__ __forceinline__ uint4 fta_lds_tr(uint32_t lo_addr, uint32_t hi_addr) {
+    const fta_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((fta_lds_s16x4*)lo_addr);
+    const fta_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((fta_lds_s16x4*)hi_addr);
+    const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
+    return make_uint4(l2.x, l2.y, h2.x, h2.y);
+}
+
 // One wave-wide LDS DMA: lane l copies 16 (or 4) bytes from g to lds + 16 * l
 // (or 4 * l).  `lds` must be wave-uniform.  Completion is tracked by vmcnt and
 // waited for explicitly (fta_wait_vmcnt + barrier).  Issued through inline asm

@@ -1,0 +1,66 @@
+"""Edges of the pipelined attention walks: blocks of several chunks, lists of one
+block, tiles that skip blocks of their workgroup's union, unsplit grids, and
+token strides past the gathers' 32-bit lane offsets."""
+
+import numpy as np
+import pytest
+import torch
+
+from _helpers import rand, say
+from test_gpu_parity import _random_merged, check_attn_vs_oracle
+
+pytestmark = pytest.mark.gpu
+
+fta = pytest.importorskip("flash_topk_attn_v2")
+
+WALK_CASES = [
+    # B, N, H, D, g, b, q padding, kv padding, W, dtype
+    (1, 500, 2, 64, 32, 160, (0, 12), (100, 40), 3, torch.float16),  # 3 chunks a block, the last of 32 keys
+    (1, 500, 2, 128, 16, 130, (4, 8), (0, 20), 2, torch.bfloat16),  # the last chunk of 2 keys
+    (1, 300, 2, 64, 16, 64, (0, 4), (0, 20), 1, torch.bfloat16),  # lists of one block: tiles skip most steps
+    (1, 300, 2, 128, 16, 64, (0, 4), (0, 20), 1, torch.float16),
+    (2, 1030, 16, 64, 64, 64, (60, 62), (63, 59), 6, torch.float16),  # unsplit grids (160 workgroups)
+    (2, 1030, 16, 128, 48, 40, (0, 26), (0, 10), 5, torch.bfloat16),
+    (1, 33, 2, 64, 33, 64, (0, 0), (31, 0), 1, torch.bfloat16),  # one block, two query tiles
+]
+
+
+@pytest.mark.parametrize("case", WALK_CASES, ids=lambda c: f"B{c[0]}N{c[1]}D{c[3]}g{c[4]}b{c[5]}W{c[8]}")
+def test_walk_edges(case):
+    B, N, H, D, g, b, qpad, kvpad, W, dt = case
+    say(f"[walk] {case}")
+    QM, M = (qpad[0] + N + qpad[1]) // g, (kvpad[0] + N + kvpad[1]) // b
+    merged = _random_merged(B, H, QM, W, M, 11)
+    q, k, v = (rand((B, N, H * D), 12 + i, dt, "cuda").requires_grad_(True) for i in range(3))
+    tm = torch.from_numpy(merged).cuda()
+    o, lse = fta.flash_topk_attn(q, k, v, tm, (tm >= 0).sum(-1).int(), H, g, b, None, None, kvpad, qpad)
+    do = rand((B, N, H * D), 99, dt, "cuda")
+    o.backward(do)
+    torch.cuda.synchronize()
+    check_attn_vs_oracle(q, k, v, do, o, lse, merged, H, g, b, qpad, kvpad, dt)
+
+
+@pytest.mark.parametrize("D,b", [(64, 64), (128, 64), (256, 64)])
+def test_wide_token_strides(D, b):
+    """Rows 2^24 + 8 elements apart run on the register-staged kernels; the same sums,
+    so o and the gradients are within one bf16 rounding step of the contiguous call."""
+    N, H, g, W = 40, 1, 16, 1
+    say(f"[wide strides] D{D}")
+    stride = 2**24 + 8
+    merged = torch.zeros(1, H, 3, W, dtype=torch.int32, device="cuda")
+    narrow = [rand((1, N, H * D), 30 + i, torch.bfloat16, "cuda") for i in range(4)]
+    wide = []
+    for t in narrow:
+        big = torch.empty((N - 1) * stride + H * D, dtype=t.dtype, device="cuda")
+        w = big.as_strided(t.shape, (N * stride, stride, 1))
+        wide.append(w.copy_(t))
+    res = []
+    for q, k, v, do in (narrow, wide):
+        q, k, v = (x.detach().requires_grad_(True) for x in (q, k, v))
+        o, lse = fta.flash_topk_attn(q, k, v, merged, None, H, g, b, None, None, (0, 24), (0, 8))
+        res.append([o.detach(), lse, *torch.autograd.grad(o, (q, k, v), do)])
+    torch.cuda.synchronize()
+    for name, x, y in zip(("o", "lse", "dq", "dk", "dv"), *res):
+        x, y = x.float().cpu().numpy(), y.float().cpu().numpy()
+        step = np.maximum(np.abs(x), np.abs(y)) * 2.0**-7 + np.abs(x).max() * 2.0**-16
+        assert (np.abs(x - y) <= step).all(), name
