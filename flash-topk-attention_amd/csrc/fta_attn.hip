@@ -1332,9 +1332,9 @@ __device__ bool fta_stage_kv_bits(const AttnArgs& a, int bh, int wk, int Tb, uin
 // Column masks of the WG's TT key tiles over 32-query chunks [seg0, seg0 + segn)
 // (tile t x chunk cl -> bits over the chunk's 32 queries), then the ascending
 // list of chunks any tile needs.  Returns the list length.
-template <int TT>
+template <int TT, int SEG, typename LT>
 __device__ int fta_build_kv_masks(const AttnArgs& a, int bh, int wk, int Tb, int seg0, int segn, bool bits_lds,
-                                  const uint32_t (*sBits)[kBitsW], uint32_t (*sMask)[kSegC], int* sList,
+                                  const uint32_t (*sBits)[kBitsW], uint32_t (*sMask)[SEG], LT* sList,
                                   int* s_tmp) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int NTHR = blockDim.x, NW = NTHR >> 6;
@@ -1394,7 +1394,7 @@ __device__ int fta_build_kv_masks(const AttnArgs& a, int bh, int wk, int Tb, int
             if (w < wave) wbase += t;
             tot += t;
         }
-        if (any) sList[U + wbase + x - any] = cl;
+        if (any) sList[U + wbase + x - any] = (LT)cl;
         __syncthreads();
         U += tot;
     }
@@ -1521,7 +1521,7 @@ __global__ __launch_bounds__(TT * CS * 64, 1) void fta_sparse_dkv_kernel(AttnArg
         const bool bits_lds = fta_stage_kv_bits<TT>(a, bh, wk, Tb, sBits);
         for (int seg0 = 0; seg0 < a.NC; seg0 += kSegC) {
             const int segn = min(kSegC, a.NC - seg0);
-            const int U = fta_build_kv_masks<TT>(a, bh, wk, Tb, seg0, segn, bits_lds, sBits, sMask, sList, s_tmp);
+            const int U = fta_build_kv_masks<TT, kSegC>(a, bh, wk, Tb, seg0, segn, bits_lds, sBits, sMask, sList, s_tmp);
             if (U == 0) continue;
             const int nsteps = (U + CS - 1) / CS;
 
@@ -1725,12 +1725,22 @@ __global__ __launch_bounds__(TT * CS * 64, 1) void fta_sparse_dkv_kernel(AttnArg
 // P crosses once, in fp32, so dS is formed from the same fp32 P as with one
 // wave per tile.  Each wave evaluates only its own half of the elementwise work
 // (the exponentials or the dS products), one of K / V and one set of
-// accumulators, so a WG fits twice on a CU (registers <= 256 per lane, LDS <
-// 80 KB): one WG's mask building and gather latency overlap the other's MFMAs.
-// At D = 256 (twice the stage bytes and accumulators) one WG runs per CU, with
-// the accumulators in the 512-register budget of one wave per SIMD.
-// One chunk per step; NST steps of Q, dO, lse and delta in flight through LDS
-// DMA, as in fta_sparse_dkv_kernel.
+// accumulators, so several WGs fit on a CU (three at D = 64, two at D = 128, with
+// registers <= 256 per lane): one WG's mask building and gather latency overlap the
+// others' MFMAs.  At D = 256 (twice the tile bytes and accumulators) one WG runs per
+// CU, with the accumulators in the 512-register budget of one wave per SIMD.
+//
+// Steps: one chunk per step and one barrier.  Role 1 works one chunk behind role 0,
+// so of the chunk in flight only Q is needed early: four Q and three dO tiles hold
+// the live chunks and two steps of gathers, in the LDS that three whole stages and
+// longer mask segments took for one step of gathers.  The list entry and mask of the
+// next step are read one step ahead, P crosses as 16-byte LDS accesses, and the rows
+// a partly selected chunk leaves out are masked with one sign-extended bit each.
+// What bounds it: each chunk's 16 KB (D = 128) serves only 64 keys, so the gathers
+// (7.4 TB/s from L2 on dense lists) and the matrix pipe (40% busy) share the time.
+// dK/dV on B1 N16384 H16 D128 dense lists 4.41 -> 4.12 ms, B1 N32768 H32 D128 short
+// lists 1.93 -> 1.81 ms, B2 N10000 H12/4 D64 g16 2.23 -> 1.58 ms (most of it from the
+// third WG per CU), N2048 H8 D256 0.118 -> 0.109 ms.
 // ----------------------------------------------------------------------------
 template <int D>
 struct DkvSplitShape {
@@ -1738,15 +1748,14 @@ struct DkvSplitShape {
     static constexpr int NTHR = 256;
     static constexpr int QSEG = D / 8;
     static constexpr int TILE = 32 * QSEG;              // 16-byte slots per 32-row tile
-    static constexpr int LQ = 2 * TILE / NTHR;          // DMA instructions per wave per step (Q, dO)
-    static constexpr int L = LQ + 1;                    // + lse / delta (wave 0)
-    static constexpr int LD_OFF = 2 * TILE * 16;        // byte offset of lse / delta in a step
-    static constexpr int STAGE_B = LD_OFF + 256;
-    static constexpr int NST = (D <= 64) ? 4 : 3;
-    static constexpr int WPC = (D <= 128) ? 2 : 1;  // WGs per CU
-    static_assert(2 * TILE % NTHR == 0, "whole DMA instructions per wave");
-    static_assert(NST >= 3, "steps k - 1 and k live, at least one in flight");
-    static_assert(NST * STAGE_B + 2 * 2 * 32 * 32 * 4 + 3 * kSegC * 4 + 2 * kBitsW * 4 + 64 <= 160 * 1024 / WPC,
+    static constexpr int LQ = TILE / NTHR;              // DMA instructions per wave per tile
+    static constexpr int TILE_B = TILE * 16;
+    static constexpr int NQ = 4, ND = 3;                // Q and dO tiles in LDS
+    static constexpr int WPC = (D <= 64) ? 3 : (D <= 128) ? 2 : 1;  // WGs per CU
+    static constexpr int SEG = 512;                     // chunks per mask segment
+    static_assert(TILE % NTHR == 0, "whole DMA instructions per wave");
+    static_assert((NQ + ND) * TILE_B + NQ * 256 + 2 * 2 * 32 * 32 * 4 + 2 * SEG * 4 + SEG * 2 + 2 * kBitsW * 4 + 64 <=
+                      160 * 1024 / WPC,
                   "WPC WGs per CU");
 };
 
@@ -1754,18 +1763,17 @@ template <int DT, int D, bool GQA, bool SPLIT>
 __global__ __launch_bounds__(256, DkvSplitShape<D>::WPC) void fta_sparse_dkv_split_kernel(AttnArgs a) {
     using E = Elem<DT>;
     using Sh = DkvSplitShape<D>;
-    constexpr int NW = Sh::NW, QSEG = Sh::QSEG, TILE = Sh::TILE, LQ = Sh::LQ, NST = Sh::NST;
-    // the 8-row swizzle (V = 1): this kernel ran 2-3% faster with it than with the
-    // conflict-free 16-row one, measured (C3 / C3-iid backward), despite its 2-way
-    // conflicts on the 16-byte operand reads
-    using SW = FtaSwz<QSEG, 1>;
+    constexpr int NW = Sh::NW, QSEG = Sh::QSEG, TILE = Sh::TILE, LQ = Sh::LQ, TILE_B = Sh::TILE_B, SEG = Sh::SEG;
+    using SW = FtaSwz<QSEG>;
     constexpr int KS = D / 16;
     constexpr int DT32 = D / 32;  // 32-column d tiles
     constexpr int TT = 2;
-    __shared__ __align__(1024) unsigned char sStage[NST][Sh::STAGE_B];
-    __shared__ float sX[2][TT][16][64];  // [step parity][tile][i][lane]: P of the last two steps
-    __shared__ uint32_t sMask[TT][kSegC];
-    __shared__ int sList[kSegC];
+    __shared__ __align__(1024) unsigned char sQ[Sh::NQ][TILE_B];
+    __shared__ __align__(1024) unsigned char sD[Sh::ND][TILE_B];
+    __shared__ __align__(1024) float sL[Sh::NQ][64];  // [lse of chunk k, delta of chunk k - 1] at k % 4
+    __shared__ float4 sX[2][TT][4][64];  // [step parity][tile][i / 4][lane]: P of the last two steps
+    __shared__ uint32_t sMask[TT][SEG];
+    __shared__ uint16_t sList[SEG];
     __shared__ uint32_t sBits[TT][kBitsW];
     __shared__ int s_tmp[8];
 
@@ -1789,7 +1797,7 @@ __global__ __launch_bounds__(256, DkvSplitShape<D>::WPC) void fta_sparse_dkv_spl
     const int hf = lane >> 5;
     const int tt = wave & 1;
     const bool hv = (wave >> 1) != 0;  // wave-uniform role: false = K / P / dV, true = V / dS / dK
-    const int Tb = 2;
+    constexpr int Tb = 2;
 
     const int krel = 32 * tt + (lane & 31);  // key of this lane's column, relative to block start
     const int tk = wk * a.kvb - a.kv_pad + krel;
@@ -1817,26 +1825,31 @@ __global__ __launch_bounds__(256, DkvSplitShape<D>::WPC) void fta_sparse_dkv_spl
     // complete the register loads: the DMAs below are invisible to the compiler
     fta_wait_vmcnt<0>();
 
-    // Per-lane DMA sources (as in fta_sparse_dkv_kernel with one chunk slot):
-    // instruction i of this wave fills 1 KB block blk = i * NW + wave of the
-    // [Q tile][dO tile] step; roff[i] = row * stride + column, in bytes.
-    int64_t roff[LQ];
+    // Per-lane DMA sources: instruction i of this wave fills 1 KB block i * NW + wave
+    // of a Q or dO tile; qoff / doff = row * stride + column, in bytes (strides <= 2^24)
+    uint32_t qoff[LQ], doff[LQ];
 #pragma unroll
     for (int i = 0; i < LQ; ++i) {
-        const int blk = i * NW + wave;
-        const int ten = (blk * 64) / TILE;
-        const int r2 = (blk * 64 + lane) % TILE;
+        const int r2 = (i * NW + wave) * 64 + lane;
         const int row = r2 / QSEG;
         int j = SW::slot(row, r2 - row * QSEG);
         if (j * 8 >= a.Dreal) j = 0;  // columns past D: any finite data (never stored)
-        roff[i] = 2 * ((int64_t)row * (ten == 1 ? a.d_sn : a.q_sn) + j * 8);
+        qoff[i] = 2u * (row * (uint32_t)a.q_sn + j * 8);
+        doff[i] = 2u * (row * (uint32_t)a.d_sn + j * 8);
     }
     // lse / delta: wave 0's DMA writes [lse 32][delta 32] (256 bytes)
     const int lv = wave * 64 + lane;
     const bool l_isd = lv >= 32 && lv < 64;
     const float* l_base = nullptr;
     const int l_row = lv & 31;
-    const uint32_t lds0 = fta_lds_addr(&sStage[0][0]);
+    // per-lane byte offsets of the operand fragments in a tile: rows of Q or dO (A
+    // operand of S / dP; other k slices by XOR of the slot bits) and transposed dO or
+    // Q (B operand of dV / dK; other column tiles by XOR, 16 rows down a constant)
+    const uint32_t aro = 2u * SW::off(lane & 31, hf);
+    const int br = 4 * (lane >> 5) + ((lane & 15) >> 2), bc = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    const uint32_t bro = 2u * (SW::off(br, bc >> 3) + (bc & 7));
+    const uint32_t bro8 = 2u * (SW::off(br + 8, bc >> 3) + (bc & 7)) - bro;  // added: rows + 8
+    const uint32_t ldq = fta_lds_addr(&sQ[0][0]), ldd = fta_lds_addr(&sD[0][0]), ldl = fta_lds_addr(&sL[0][0]);
 
     // the rest runs in one copy per role, so each keeps only its own values live
     auto run = [&](auto role) {
@@ -1862,9 +1875,9 @@ __global__ __launch_bounds__(256, DkvSplitShape<D>::WPC) void fta_sparse_dkv_spl
                 __syncthreads();  // the previous head's membership rows are no longer read
                 bits_lds = fta_stage_kv_bits<TT>(a, bh, wk, Tb, sBits);
             }
-            for (int seg0 = 0; seg0 < a.NC; seg0 += kSegC) {
-                const int segn = min(kSegC, a.NC - seg0);
-                const int Ua = fta_build_kv_masks<TT>(a, bh, wk, Tb, seg0, segn, bits_lds, sBits, sMask, sList, s_tmp);
+            for (int seg0 = 0; seg0 < a.NC; seg0 += SEG) {
+                const int segn = min(SEG, a.NC - seg0);
+                const int Ua = fta_build_kv_masks<TT, SEG>(a, bh, wk, Tb, seg0, segn, bits_lds, sBits, sMask, sList, s_tmp);
                 // this part's chunk-list positions [u_lo, u_lo + U) (workgroup-uniform)
                 int u_lo = 0, U = Ua;
                 if constexpr (SPLIT) {
@@ -1873,155 +1886,192 @@ __global__ __launch_bounds__(256, DkvSplitShape<D>::WPC) void fta_sparse_dkv_spl
                 }
                 // no wave reads sMask / sList below when the part is empty
                 if (U == 0) continue;
-                const int* lst = sList + u_lo;
+                const uint16_t* lst = sList + u_lo;
 
-                // gather chunk list entry k into stage buffer st
-                auto issue = [&](int st, int k) {
-                    const uint32_t sbase = lds0 + st * Sh::STAGE_B;
-                    const int c = __builtin_amdgcn_readfirstlane(seg0 + lst[k]);
+                // gather one tile of a tensor: chunk c's 32 rows to LDS address lds
+                auto tile = [&](const uint16_t* base, int64_t sn, const uint32_t* off, int c, uint32_t lds)
+                    __attribute__((always_inline)) {
                     const int t0 = 32 * c - a.q_pad;
+                    const int tb = min(max(t0, 0), a.N - 1);
+                    const uint16_t* bp = base + (int64_t)tb * sn;
                     if (t0 >= 0 && t0 + 31 < a.N) {
 #pragma unroll
-                        for (int i = 0; i < LQ; ++i) {
-                            const int blk = i * NW + wave;
-                            const int ten = (blk * 64) / TILE;
-                            const char* base =
-                                reinterpret_cast<const char*>(ten == 1 ? dp + (int64_t)t0 * a.d_sn : qp + (int64_t)t0 * a.q_sn);
-                            fta_dma16_at(base + roff[i], sbase + blk * 1024);
-                        }
+                        for (int i = 0; i < LQ; ++i) fta_dma16_so(bp, off[i], lds + (i * NW + wave) * 1024);
                     } else {  // a chunk at a sequence edge: clamp its rows (masked off) into [0, N)
 #pragma unroll
                         for (int i = 0; i < LQ; ++i) {
-                            const int blk = i * NW + wave;
-                            const int ten = (blk * 64) / TILE;
-                            const int r2 = (blk * 64 + lane) % TILE;
+                            const int r2 = (i * NW + wave) * 64 + lane;
                             const int row = r2 / QSEG;
                             int j = SW::slot(row, r2 - row * QSEG);
                             if (j * 8 >= a.Dreal) j = 0;
-                            const int t = min(max(t0 + row, 0), a.N - 1);
-                            fta_dma16_at((ten == 1 ? dp + (int64_t)t * a.d_sn : qp + (int64_t)t * a.q_sn) + j * 8,
-                                         sbase + blk * 1024);
+                            const uint32_t rel = (uint32_t)(min(max(t0 + row, 0), a.N - 1) - tb);  // 0 .. 31
+                            fta_dma16_so(bp, 2u * (rel * (uint32_t)sn + j * 8), lds + (i * NW + wave) * 1024);
                         }
                     }
-                    if (wave == 0) {  // lse and delta of the chunk's 32 rows: one 256-byte DMA
-                        const int t = min(max(t0 + l_row, 0), a.N - 1);
-                        fta_dma4_at(l_base + t, sbase + Sh::LD_OFF);
+                };
+                // step kq - 2's gathers: Q and lse of chunk cq (list entry kq), dO and delta
+                // of chunk cd (entry kq - 1)
+                auto issue = [&](int kq, int dslot, int cq, int cd) __attribute__((always_inline)) {
+                    tile(qp, a.q_sn, qoff, cq, ldq + (kq & 3) * TILE_B);
+                    tile(dp, a.d_sn, doff, cd, ldd + dslot * TILE_B);
+                    if (wave == 0) {
+                        const int t = min(max(32 * (l_isd ? cd : cq) - a.q_pad + l_row, 0), a.N - 1);
+                        fta_dma4_at(l_base + t, ldl + (kq & 3) * 256);
                     }
                 };
 
-                // Software pipeline, one barrier per step: iteration k computes S_k / P_k
-                // and dV_k (role 0) and dP_k (role 1); role 1 forms dS_{k-1} from P_{k-1}
-                // (written to LDS in iteration k - 1) and adds dK_{k-1}, so the stage
-                // buffers of steps k - 1 and k are live and NST - 2 steps are in flight.
-#pragma unroll
-                for (int k = 0; k < NST - 2; ++k)
-                    if (k < U) issue(k, k);
-                int cur = 0;       // stage buffer of step k
-                bool pm = false;   // step k - 1 left its accumulation (dV or dK) to do
-                f32x16 dpp;        // role 1: dP_{k-1}
-                uint4 af[2];       // A operand of that accumulation: P_{k-1} (role 0) or dS_{k-1} (role 1)
+                // One barrier per step.  Step k: role 0 computes S_k / P_k (P_k to LDS) and
+                // adds dV_{k-1}; role 1 takes chunk k - 1 whole: dP, dS (P from LDS), dK.
+                // Live: Q of chunks k - 1 and k, dO of k - 1; two steps of gathers are in
+                // flight (Q of k + 1 and k + 2, dO of k and k + 1).  Gathers past the list
+                // repeat its last chunk, so every step issues the same number.
+                const int last = U - 1;
+                int c1 = __builtin_amdgcn_readfirstlane((int)lst[0]);
+                uint32_t mk = __builtin_amdgcn_readfirstlane(sMask[tt][c1]), mkp = 0u;
+                issue(0, 2, seg0 + c1, seg0 + c1);
+                int c2 = __builtin_amdgcn_readfirstlane((int)lst[min(1, last)]);
+                issue(1, 0, seg0 + c2, seg0 + c1);
+                c1 = c2;                                                     // entry k + 1
+                c2 = __builtin_amdgcn_readfirstlane((int)lst[min(2, last)]);  // entry k + 2
+                int ds = 2;       // dO slot of chunk k - 1
+                uint4 af[2];      // role 0: P_{k-1}, A operand of dV_{k-1}
                 for (int k = 0; k <= U; ++k) {
-                    if (k + NST - 3 >= U)
-                        fta_wait_vmcnt<0>();
-                    else if (wave == 0)  // wave 0 issues the lse / delta DMA as well
-                        fta_wait_vmcnt<Sh::L * (NST - 3)>();
+                    // step k - 2's gathers complete (wave 0 issues the lse / delta DMA as well)
+                    if (wave == 0)
+                        fta_wait_vmcnt<2 * LQ + 1>();
                     else
-                        fta_wait_vmcnt<(Sh::L - 1) * (NST - 3)>();
-                    // step k visible; step k - 2's buffer is free; P_{k-1} visible, sX[k & 1] free
+                        fta_wait_vmcnt<2 * LQ>();
+                    // Q_k, dO_{k-1} and P_{k-1} visible; the slots of Q_{k-2}, dO_{k-2} and sX[k & 1] free
                     __syncthreads();
-                    if (k + NST - 2 < U) issue(cur >= 2 ? cur - 2 : cur + NST - 2, k + NST - 2);
-                    const int prv = cur == 0 ? NST - 1 : cur - 1;  // stage buffer of step k - 1
-                    const uint32_t mk = (k < U) ? __builtin_amdgcn_readfirstlane(sMask[tt][lst[k]]) : 0u;
-                    const uint16_t* qb = reinterpret_cast<const uint16_t*>(&sStage[cur][0]);
-                    const uint16_t* ob = qb + TILE * 8;
-                    const float* ld = reinterpret_cast<const float*>(&sStage[cur][Sh::LD_OFF]);
-                    // B operand of step k - 1's accumulation: dO^T (role 0, dV) or Q^T (role 1, dK)
-                    const uint16_t* bb1 =
-                        reinterpret_cast<const uint16_t*>(&sStage[pm ? prv : cur][0]) + (HV ? 0 : TILE * 8);
-                    if (!pm) af[0] = af[1] = fta_zero4();
-                    if (HV && pm) {  // dS_{k-1} = P_{k-1} (dP_{k-1} - delta)
-                        const float* ld1 = reinterpret_cast<const float*>(&sStage[prv][Sh::LD_OFF]);
+                    issue(k + 2, ds == 0 ? 2 : ds - 1, seg0 + c2, seg0 + c1);
+                    const uint32_t v_mk = sMask[tt][c1];
+                    const int v_c = lst[min(k + 3, last)];
+                    const float* ld = &sL[k & 3][0];
+                    const uint32_t dbase = ldd + ds * TILE_B;
+                    if constexpr (!HV) {
+                        const uint32_t qb = ldq + (k & 3) * TILE_B + aro, ob = dbase + bro;
+                        const bool pm = mkp != 0u;
+                        if (!pm) af[0] = af[1] = fta_zero4();
+                        // S_k (a dependent chain) interleaved with dV_{k-1} (independent MFMAs).
+                        // One instruction stream for every case: without a pending accumulation
+                        // P is zero and dO any finite tile (acc += 0 exactly); without a chain
+                        // the S result is discarded.
+                        if (mk | mkp) {
+                            f32x16 own;  // S_k then P_k
+#pragma unroll
+                            for (int i = 0; i < 16; ++i) own[i] = 0.f;
+                            uint4 fs[2], fa2[2];
+                            auto load = [&](int j, int slot) {
+                                fs[slot] = fta_lds_b128(qb ^ (j * 32));
+                                const uint32_t x = (j / DT32) * 16 * QSEG * 16;
+                                fa2[slot] = fta_lds_tr((ob ^ ((j % DT32) * 64)) + x, ((ob + bro8) ^ ((j % DT32) * 64)) + x);
+                            };
+                            load(0, 0);
+#pragma unroll
+                            for (int j = 0; j < KS; ++j) {  // KS = 2 * DT32: one accumulation MFMA per chain link
+                                if (j + 1 < KS) load(j + 1, (j + 1) & 1);
+                                own = E::mma(fs[j & 1], kv[j], own);
+                                acc[j % DT32] = E::mma(af[j / DT32], fa2[j & 1], acc[j % DT32]);
+                            }
+                            __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+#pragma unroll
+                            for (int j = 0; j < KS; ++j) {
+                                if (j + 1 < KS) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+                                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                            }
+                            if (mk) {  // P_k = 2^{c S_k - lse2}: to LDS for role 1, packed for dV_k
+                                if (mk == 0xffffffffu && __ballot(!kok) == 0ull) {
+                                    // every row of the chunk selected, every key valid: no mask
+#pragma unroll
+                                    for (int i = 0; i < 16; ++i)
+                                        own[i] = fta_exp2(fmaf(own[i], a.c, -ld[c_row(i, lane)]));
+                                } else {
+                                    // row c_row(i, lane) is bit (i >> 2) * 8 + (i & 3) of mk >> 4 hf; a
+                                    // selected row with a valid key has a finite lse
+                                    const uint32_t ml = kok ? mk >> (4 * hf) : 0u;
+#pragma unroll
+                                    for (int i = 0; i < 16; ++i) {
+                                        const float ex = fta_exp2(fmaf(own[i], a.c, -ld[c_row(i, lane)]));
+                                        const int keep = ((int)(ml << (31 - ((i >> 2) * 8 + (i & 3))))) >> 31;
+                                        own[i] = __builtin_bit_cast(float, __builtin_bit_cast(int, ex) & keep);
+                                    }
+                                }
+#pragma unroll
+                                for (int i = 0; i < 16; i += 4)
+                                    sX[k & 1][tt][i / 4][lane] = make_float4(own[i], own[i + 1], own[i + 2], own[i + 3]);
+#pragma unroll
+                                for (int ks = 0; ks < 2; ++ks)
+                                    af[ks] = make_uint4(E::pack2(own[8 * ks], own[8 * ks + 1]),
+                                                        E::pack2(own[8 * ks + 2], own[8 * ks + 3]),
+                                                        E::pack2(own[8 * ks + 4], own[8 * ks + 5]),
+                                                        E::pack2(own[8 * ks + 6], own[8 * ks + 7]));
+                            }
+                        }
+                    } else if (mkp) {
+                        const uint32_t ob = dbase + aro, qb = ldq + ((k + 3) & 3) * TILE_B + bro;
+                        f32x16 dpv;
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) dpv[i] = 0.f;
+                        {
+                            constexpr int PD = 3;
+                            uint4 fr[PD + 1];
+                            auto load = [&](auto nn) __attribute__((always_inline)) {
+                                constexpr int n = decltype(nn)::value;
+                                if constexpr (n < KS) fr[n % (PD + 1)] = fta_lds_b128(ob ^ (n * 32));
+                            };
+                            auto slot = [&](auto nn) __attribute__((always_inline)) {
+                                constexpr int n = decltype(nn)::value;
+                                load(std::integral_constant<int, n + PD>{});
+                                dpv = E::mma(fr[n % (PD + 1)], kv[n], dpv);
+                            };
+                            fta_for<0, PD>(load);
+                            fta_for<0, KS>(slot);
+                        }
+                        uint4 ds2[2];  // dS = P (dP - delta)
 #pragma unroll
                         for (int ks = 0; ks < 2; ++ks) {
                             float dv8[8];
 #pragma unroll
-                            for (int e = 0; e < 8; ++e) {
+                            for (int e = 0; e < 8; e += 4) {
                                 const int i = 8 * ks + e;
-                                dv8[e] = sX[(k + 1) & 1][tt][i][lane] * (dpp[i] - ld1[32 + c_row(i, lane)]);
+                                const float4 pr = sX[(k + 1) & 1][tt][i / 4][lane];
+                                const float4 dl = *reinterpret_cast<const float4*>(ld + 32 + c_row(i, lane));
+                                dv8[e] = pr.x * (dpv[i] - dl.x);
+                                dv8[e + 1] = pr.y * (dpv[i + 1] - dl.y);
+                                dv8[e + 2] = pr.z * (dpv[i + 2] - dl.z);
+                                dv8[e + 3] = pr.w * (dpv[i + 3] - dl.w);
                             }
-                            af[ks] = make_uint4(E::pack2(dv8[0], dv8[1]), E::pack2(dv8[2], dv8[3]),
-                                                E::pack2(dv8[4], dv8[5]), E::pack2(dv8[6], dv8[7]));
+                            ds2[ks] = make_uint4(E::pack2(dv8[0], dv8[1]), E::pack2(dv8[2], dv8[3]),
+                                                 E::pack2(dv8[4], dv8[5]), E::pack2(dv8[6], dv8[7]));
                         }
-                    }
-                    // S_k / dP_k (a dependent chain) interleaved with step k - 1's
-                    // accumulation (independent MFMAs): the matrix pipe stays fed
-                    f32x16 own;  // S_k then P_k (role 0) or dP_k (role 1)
-                    const uint16_t* ab = HV ? ob : qb;
-                    auto mmas = [&](auto with_s, auto with_acc) {
-                        constexpr bool WS = decltype(with_s)::value, WA = decltype(with_acc)::value;
-                        if (WS) {
-#pragma unroll
-                            for (int i = 0; i < 16; ++i) own[i] = 0.f;
-                        }
-                        // fragments of link j + 1 load while link j's MFMAs run
-                        uint4 fs[2], fa2[2];
-                        auto load = [&](int j, int slot) {
-                            if (WS) fs[slot] = *reinterpret_cast<const uint4*>(ab + SW::off(lane & 31, 2 * j + hf));
-                            if (WA) fa2[slot] = fta_tr_frag_sw<QSEG, 1>(bb1, (j / DT32) * 16, (j % DT32) * 32, lane);
-                        };
-                        constexpr int NR = (WS ? 1 : 0) + (WA ? 2 : 0);  // LDS reads per link
-                        constexpr int NM = (WS ? 1 : 0) + (WA ? 1 : 0);  // MFMAs per link
-                        load(0, 0);
-#pragma unroll
-                        for (int j = 0; j < KS; ++j) {  // KS = 2 * DT32: one accumulation MFMA per chain link
-                            if (j + 1 < KS) load(j + 1, (j + 1) & 1);
-                            if (WS) own = E::mma(fs[j & 1], kv[j], own);
-                            if (WA) acc[j % DT32] = E::mma(af[j / DT32], fa2[j & 1], acc[j % DT32]);
-                        }
-                        __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);
-#pragma unroll
-                        for (int j = 0; j < KS; ++j) {
-                            if (j + 1 < KS) __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);
-                            __builtin_amdgcn_sched_group_barrier(0x008, NM, 0);
-                        }
-                    };
-                    // One instruction stream for every case (separate variants cost the
-                    // register budget): without a pending accumulation the A operand is zero
-                    // and the B operand the current step's finite data (acc += 0 exactly);
-                    // without a chain the S / dP result is discarded.
-                    if (mk || pm) mmas(std::true_type{}, std::true_type{});
-                    if (mk) {
-                        if (!HV) {  // P_k = 2^{c S_k - lse2}: to LDS for role 1, packed for dV_k
-                            if (mk == 0xffffffffu && __ballot(!kok) == 0ull) {
-                                // every row of the chunk selected, every key valid: no mask
-#pragma unroll
-                                for (int i = 0; i < 16; ++i) own[i] = fta_exp2(fmaf(own[i], a.c, -ld[c_row(i, lane)]));
-                            } else {
-#pragma unroll
-                                for (int i = 0; i < 16; ++i) {
-                                    const int r = c_row(i, lane);
-                                    // a selected row with a valid key has a finite lse
-                                    const bool ok = kok && ((mk >> r) & 1u);
-                                    const float ex = fta_exp2(fmaf(own[i], a.c, -ld[r]));
-                                    own[i] = ok ? ex : 0.f;
+                        {
+                            constexpr int PD = 3;
+                            uint4 fr[PD + 1];
+                            auto load = [&](auto nn) __attribute__((always_inline)) {
+                                constexpr int n = decltype(nn)::value;
+                                if constexpr (n < KS) {
+                                    constexpr int x = (n / DT32) * 16 * QSEG * 16;
+                                    fr[n % (PD + 1)] = fta_lds_tr((qb ^ ((n % DT32) * 64)) + x,
+                                                                  ((qb + bro8) ^ ((n % DT32) * 64)) + x);
                                 }
-                            }
-#pragma unroll
-                            for (int i = 0; i < 16; ++i) sX[k & 1][tt][i][lane] = own[i];
-#pragma unroll
-                            for (int ks = 0; ks < 2; ++ks)
-                                af[ks] = make_uint4(E::pack2(own[8 * ks], own[8 * ks + 1]),
-                                                    E::pack2(own[8 * ks + 2], own[8 * ks + 3]),
-                                                    E::pack2(own[8 * ks + 4], own[8 * ks + 5]),
-                                                    E::pack2(own[8 * ks + 6], own[8 * ks + 7]));
-                        } else {
-                            dpp = own;
+                            };
+                            auto slot = [&](auto nn) __attribute__((always_inline)) {
+                                constexpr int n = decltype(nn)::value;
+                                load(std::integral_constant<int, n + PD>{});
+                                acc[n % DT32] = E::mma(ds2[n / DT32], fr[n % (PD + 1)], acc[n % DT32]);
+                            };
+                            fta_for<0, PD>(load);
+                            fta_for<0, KS>(slot);
                         }
                     }
-                    pm = mk != 0u;
-                    cur = (cur == NST - 1) ? 0 : cur + 1;
+                    mkp = mk;
+                    c1 = c2;
+                    c2 = __builtin_amdgcn_readfirstlane(v_c);
+                    mk = (k + 1 < U) ? __builtin_amdgcn_readfirstlane(v_mk) : 0u;
+                    ds = (ds == 2) ? 0 : ds + 1;
                 }
-                __syncthreads();  // all waves done with the stage buffers, sMask and sList
+                fta_wait_vmcnt<0>();  // the gathers past the list's end
+                __syncthreads();      // all waves done with the tiles, sMask and sList
             }
         }
 
@@ -2270,6 +2320,8 @@ int launch_dq_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
 template <int DT>
 int launch_dkv_dt(AttnArgs& a, int Dk, int Tb, int B, int H, int ntiles, hipStream_t st) {
     const bool gqa = a.G > 1;
+    // the split kernel keeps per-lane Q / dO row offsets in 32 bits
+    const bool split_ok = Tb == 2 && narrow_stride(a.q_sn) && narrow_stride(a.d_sn);
     // ns: parts per KV block (the split kernel with a.nsplit > 1), else 1
     auto go = [&](auto kern, int tt, int nw, int ns) {
         a.wg_per_bh = (ntiles + tt - 1) / tt;
@@ -2298,7 +2350,7 @@ int launch_dkv_dt(AttnArgs& a, int Dk, int Tb, int B, int H, int ntiles, hipStre
             : go(fta_sparse_dkv_split_kernel<DT, DK, false, false>, 2, 4, 1)
         FTA_DKV(32, 8, 1, 4, 2, 4)
         case 64:
-            if (Tb == 2)
+            if (split_ok)
                 FTA_DKV_SPLIT(64);
             else if (Tb == 1)
                 FTA_DKV_GO(64, 1, 4);
@@ -2307,7 +2359,7 @@ int launch_dkv_dt(AttnArgs& a, int Dk, int Tb, int B, int H, int ntiles, hipStre
             break;
         FTA_DKV(96, 4, 1, 4, 2, 2)
         case 128:
-            if (Tb == 2)
+            if (split_ok)
                 FTA_DKV_SPLIT(128);
             else if (Tb == 1)
                 FTA_DKV_GO(128, 1, 4);
@@ -2316,7 +2368,7 @@ int launch_dkv_dt(AttnArgs& a, int Dk, int Tb, int B, int H, int ntiles, hipStre
             break;
         FTA_DKV(160, 4, 2, 2, 2, 2)
         case 256:
-            if (Tb == 2)
+            if (split_ok)
                 FTA_DKV_SPLIT(256);
             else
                 FTA_DKV_GO(256, 4, 1);
@@ -2688,7 +2740,8 @@ int fta_sparse_attn_bwd_dkv(const void* q, const int64_t* q_strides, const void*
     // fta_dkv_combine_kernel, when the workspace has room for the parts
     const int ns = dkv_nsplit(B, Hk, kv_block_size, G);
     const size_t used = bwd_bytes(B, H, N, G);
-    const bool split = ns > 1 && workspace_bytes >= used + dkv_split_bytes(B, Hk, G, ns);
+    const bool split = ns > 1 && workspace_bytes >= used + dkv_split_bytes(B, Hk, G, ns) &&
+                       narrow_stride(a.q_sn) && narrow_stride(a.d_sn);
     a.nsplit = split ? ns : 1;
     a.nbh = B * Hk;
     a.npq = G.Mkv * 64;

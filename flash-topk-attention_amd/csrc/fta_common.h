@@ -136,18 +136,14 @@ __device__ __forceinline__ uint4 fta_tr_frag(const uint16_t* tile, int row, int 
 //    per C3-iid sparse forward, 5.5e8 per C3 scoring launch);
 //  * ds_read_b64_tr_b16 is served 32 lanes at a time over 256 bytes: 4
 //    consecutive rows x 64 bytes, so bits 2..3 of x must differ across them.
-// x(r) = (r & 3) << 2 | (r >> 2) & 3 meets both for 16 or more slots per row
-// (V = 1 keeps the earlier 8-row form, which one kernel measured faster with);
-// 8 slots (128-byte rows, two rows per bank line) use the row-pair form; 4
+// x(r) = (r & 3) << 2 | (r >> 2) & 3 meets both for 16 or more slots per row; 8 slots (128-byte rows, two rows per bank line) use the row-pair form; 4
 // slots need none.  12 and 20 slots use r & 3 (not tuned).
 // ---------------------------------------------------------------------------
-template <int QSEG, int V = 0>
+template <int QSEG>
 struct FtaSwz {
     static_assert(QSEG % 4 == 0, "rows must be a multiple of 4 slots");
     __device__ static __forceinline__ int x(int r) {
-        if constexpr (QSEG % 16 == 0 && V == 1) {
-            return ((r & 1) << 2) | (((r >> 1) & 1) * 10) | ((r >> 2) & 1);
-        } else if constexpr (QSEG % 16 == 0) {
+        if constexpr (QSEG % 16 == 0) {
             return ((r & 3) << 2) | ((r >> 2) & 3);
         } else if constexpr (QSEG == 8) {
             const int h = (r >> 1) & 7;
@@ -165,13 +161,13 @@ struct FtaSwz {
 };
 
 // fta_tr_frag over a swizzled tile of QSEG slots per row.
-template <int QSEG, int V = 0>
+template <int QSEG>
 __device__ __forceinline__ uint4 fta_tr_frag_sw(const uint16_t* tile, int k0, int n0, int lane) {
     const int g = lane >> 4, i = lane & 15;
     const int r = k0 + 4 * (g >> 1) + (i >> 2);
     const int col = n0 + 16 * (g & 1) + 4 * (i & 3);
-    const uint16_t* p0 = tile + FtaSwz<QSEG, V>::off(r, col >> 3) + (col & 7);
-    const uint16_t* p1 = tile + FtaSwz<QSEG, V>::off(r + 8, col >> 3) + (col & 7);
+    const uint16_t* p0 = tile + FtaSwz<QSEG>::off(r, col >> 3) + (col & 7);
+    const uint16_t* p1 = tile + FtaSwz<QSEG>::off(r + 8, col >> 3) + (col & 7);
     const fta_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
         (fta_lds_s16x4*)(__attribute__((address_space(3))) uint16_t*)p0);
     const fta_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
