@@ -28,7 +28,8 @@
 #include <type_traits>
 
 namespace fta {
-int launch_sel_bitmap(const int32_t* merged, int BH, int QM, int W, int M, uint32_t* sel, hipStream_t st);
+int launch_sel_bitmap(const int32_t* merged, int BH, int QM, int W, int M, uint32_t* sel, const float* lse,
+                      float* lse2, int64_t n_lse, hipStream_t st);
 int launch_kv_order(const uint32_t* sel, int B, int H, int Hk, int M, int QW, int32_t* order, int32_t* head_work,
                     int32_t* head_perm, hipStream_t st);
 int launch_head_order_merged(const int32_t* merged, int BH, int QM, int W, int M, int qpg, int32_t* head_work,
@@ -89,28 +90,51 @@ __device__ __forceinline__ uint32_t fta_range_bits(int lo, int hi) {
 template <int T, typename LT>
 __device__ int fta_build_q_masks(const AttnArgs& a, int bh, int p0, int seg0, int segn, uint32_t (*sMask)[kSeg],
                                  LT* sList, int* s_tmp) {
-    const int tid = threadIdx.x;
-    for (int i = tid; i < T * kSeg; i += blockDim.x) sMask[i / kSeg][i % kSeg] = 0u;
+    // opaque copies: nothing derived from them can be hoisted out of the caller's segment
+    // loop, where it would hold registers through the chunk loop (28 spills at D = 64)
+    int tid = threadIdx.x, width = a.W;
+    asm volatile("" : "+v"(tid), "+s"(width));
+    for (int i = tid; i < T * kSeg / 4; i += blockDim.x)
+        reinterpret_cast<uint4*>(&sMask[0][0])[i] = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
     const int pend = p0 + 32 * T;
     const int qb_lo = p0 / a.g;
     int qb_hi = (pend - 1) / a.g;
     if (qb_hi > a.QM - 1) qb_hi = a.QM - 1;
     const int vlo = a.q_pad, vhi = a.q_pad + a.N;  // valid padded query positions
-    const int npairs = (qb_hi - qb_lo + 1) * a.W;
-    for (int pi = tid; pi < npairs; pi += blockDim.x) {
-        const int qb = qb_lo + pi / a.W;
-        const int s = pi - (pi / a.W) * a.W;
-        const int m = a.merged[((int64_t)bh * a.QM + qb) * a.W + s];
-        if (m < seg0 || m >= seg0 + segn || m >= a.Mkv) continue;
-        int lo = qb * a.g, hi = qb * a.g + a.g;
-        lo = max(lo, max(p0, vlo));
-        hi = min(hi, min(pend, vhi));
-        if (lo >= hi) continue;
+    // rows [lo, hi) of the WG's tiles that q-block qb covers
+    auto rows_of = [&](int qb, int& lo, int& hi) {
+        lo = max(qb * a.g, max(p0, vlo));
+        hi = min(qb * a.g + a.g, min(pend, vhi));
+    };
+    auto put = [&](int m, int lo, int hi) {
+        if (m < seg0 || m >= seg0 + segn || m >= a.Mkv || lo >= hi) return;
         for (int tau = (lo - p0) >> 5; tau <= (hi - 1 - p0) >> 5; ++tau) {
             const int tb = p0 + 32 * tau;
-            const uint32_t bits = fta_range_bits(max(lo, tb) - tb, min(hi, tb + 32) - tb);
-            atomicOr(&sMask[tau][m - seg0], bits);
+            atomicOr(&sMask[tau][m - seg0], fta_range_bits(max(lo, tb) - tb, min(hi, tb + 32) - tb));
+        }
+    };
+    const int32_t* ids = a.merged + ((int64_t)bh * a.QM + qb_lo) * width;
+    const int nrow = qb_hi - qb_lo + 1;
+    if ((width & 3) == 0 && ((uintptr_t)a.merged & 15) == 0) {
+        // 16-byte loads: 8 rows of 256 ids are one load per thread instead of four in turn
+        const int w4 = width >> 2, n = nrow * w4;
+        const int4* ids4 = reinterpret_cast<const int4*>(ids);
+        for (int e = tid; e < n; e += blockDim.x) {
+            const int4 v = ids4[e];
+            int lo, hi;
+            rows_of(qb_lo + e / w4, lo, hi);
+            put(v.x, lo, hi);
+            put(v.y, lo, hi);
+            put(v.z, lo, hi);
+            put(v.w, lo, hi);
+        }
+    } else {
+        const int n = nrow * width;
+        for (int e = tid; e < n; e += blockDim.x) {
+            int lo, hi;
+            rows_of(qb_lo + e / width, lo, hi);
+            put(ids[e], lo, hi);
         }
     }
     __syncthreads();
@@ -166,7 +190,7 @@ __global__ __launch_bounds__(NW * 64, 1) void fta_sparse_fwd_kernel(AttnArgs a) 
     constexpr int KLOADS = (64 * KSEG + NTHR - 1) / NTHR;
     __shared__ __align__(16) uint16_t sK[2][64 * KROW];
     __shared__ __align__(16) uint16_t sV[2][64 * KROW];
-    __shared__ uint32_t sMask[T][kSeg];
+    __shared__ __align__(16) uint32_t sMask[T][kSeg];
     __shared__ int sList[kSeg];
     __shared__ int s_tmp[8];
 
@@ -520,7 +544,7 @@ __global__ __launch_bounds__(NW * 64, D <= 64 ? 4 : 1) void fta_sparse_fwd_pipe_
     constexpr int KS = D / 16;
     constexpr int DT32 = D / 32;
     __shared__ __align__(1024) unsigned char sStage[NST][Sh::STAGE_B];
-    __shared__ uint32_t sMask[T][kSeg];
+    __shared__ __align__(16) uint32_t sMask[T][kSeg];
     __shared__ uint16_t sList[kSeg];
     __shared__ int s_tmp[8];
 
@@ -833,7 +857,7 @@ __global__ __launch_bounds__(NW * 64, 1) void fta_sparse_dq_kernel(AttnArgs a) {
     constexpr int KLOADS = (64 * KSEG + NTHR - 1) / NTHR;
     __shared__ __align__(16) uint16_t sK[NB][64 * KROW];
     __shared__ __align__(16) uint16_t sV[NB][64 * KROW];
-    __shared__ uint32_t sMask[T][kSeg];
+    __shared__ __align__(16) uint32_t sMask[T][kSeg];
     __shared__ int sList[kSeg];
     __shared__ int s_tmp[8];
 
@@ -1045,7 +1069,7 @@ __global__ __launch_bounds__(512, 1) void fta_sparse_dq_pipe_kernel(AttnArgs a) 
     constexpr int KS = D / 16;
     constexpr int DT32 = D / 32;
     __shared__ __align__(1024) unsigned char sStage[NST][Sh::STAGE_B];
-    __shared__ uint32_t sMask[T][kSeg];
+    __shared__ __align__(16) uint32_t sMask[T][kSeg];
     __shared__ uint16_t sList[kSeg];
     __shared__ int s_tmp[8];
 
@@ -2148,13 +2172,6 @@ __global__ __launch_bounds__(256) void fta_dkv_combine_kernel(AttnArgs a) {
     *reinterpret_cast<uint2*>(op + 4) = make_uint2(E::pack2(o[4] * sc, o[5] * sc), E::pack2(o[6] * sc, o[7] * sc));
 }
 
-// lse2 = lse * log2(e) (the same fp32 product the kernels formed per element)
-__global__ __launch_bounds__(256) void fta_lse2_kernel(const float* __restrict__ lse, float* __restrict__ lse2,
-                                                       int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) lse2[i] = lse[i] * 1.4426950408889634f;
-}
-
 // ----------------------------------------------------------------------------
 // Host side
 // ----------------------------------------------------------------------------
@@ -2616,10 +2633,12 @@ int bwd_common(AttnArgs& a, Geo& G, const void* q, const int64_t* q_strides, con
 }
 
 // 64-key blocks at D 64 / 128 / 256 (the split dK/dV kernel) run in the launch
-// order of fta_kv_order_kernel and the head placement of fta_head_balance_kernel
-bool uses_kv_order(int kv_block_size, const Geo& G) {
+// order of fta_kv_order_kernel and the head placement of fta_head_balance_kernel,
+// except on grids that split (dkv_nsplit: all their workgroups run at once, so the
+// order cannot change the time; the two launches took 10 of 199 us at N2048 H8 D128)
+bool uses_kv_order(int B, int Hk, int kv_block_size, const Geo& G) {
     return kv_block_size > 32 && kv_block_size <= 64 && (G.Dk == 64 || G.Dk == 128 || G.Dk == 256) &&
-           G.Mkv <= 4096;
+           G.Mkv <= 4096 && dkv_nsplit(B, Hk, kv_block_size, G) == 1;
 }
 
 // the head placement fta_sparse_attn_bwd_dkv left in the workspace (null if it made none)
@@ -2628,7 +2647,7 @@ const int32_t* dkv_head_perm(const void* workspace, int B, int H, int N, int D, 
     Geo G;
     if (geometry(B, H, N, D, q_block_size, kv_block_size, q_pad_head, q_pad_tail, kv_pad_head, kv_pad_tail, QM, &G) !=
             FTA_OK ||
-        !uses_kv_order(kv_block_size, G))
+        !uses_kv_order(B, H, kv_block_size, G))
         return nullptr;
     const char* p = (const char*)workspace + sel_bytes(B, H, G) + fta::align_up((size_t)B * H * N * sizeof(float)) +
                     fta::align_up((size_t)B * H * G.Mkv * sizeof(int32_t));
@@ -2708,15 +2727,14 @@ int fta_sparse_attn_bwd_dkv(const void* q, const int64_t* q_strides, const void*
     hipStream_t st = (hipStream_t)stream;
     // membership bitmap (KV block -> q-blocks) and lse in log2 units, in the workspace
     uint32_t* sel = (uint32_t*)workspace;
-    if ((rc = fta::launch_sel_bitmap(merged_indices, B * H, QM, W, G.Mkv, sel, st)) != FTA_OK) return rc;
     float* lse2 = (float*)((char*)workspace + sel_bytes(B, H, G));
-    const int64_t nl = (int64_t)B * H * N;
-    hipLaunchKernelGGL(fta_lse2_kernel, dim3((unsigned)((nl + 255) / 256)), dim3(256), 0, st, lse, lse2, nl);
-    if ((rc = fta::check_launch("fta_lse2_kernel")) != FTA_OK) return rc;
+    if ((rc = fta::launch_sel_bitmap(merged_indices, B * H, QM, W, G.Mkv, sel, lse, lse2, (int64_t)B * H * N, st)) !=
+        FTA_OK)
+        return rc;
     a.sel = sel;
     a.lse2_in = lse2;
     // 64-key blocks at D 64 / 128 (the split kernel): launch in first-q-block order
-    if (uses_kv_order(kv_block_size, G)) {
+    if (uses_kv_order(B, Hk, kv_block_size, G)) {
         int32_t* order = (int32_t*)((char*)lse2 + fta::align_up((size_t)B * H * N * sizeof(float)));
         int32_t* head_work = (int32_t*)((char*)order + fta::align_up((size_t)B * H * G.Mkv * sizeof(int32_t)));
         int32_t* head_perm = head_work + B * Hk;

@@ -575,34 +575,79 @@ __global__ __launch_bounds__(256) void fta_qblock_merge_hist_kernel(
 // ids ascending) are deterministic.
 // ----------------------------------------------------------------------------
 
+// Calls f(row, id) for each of the rows x W ids at `p` (row-major), this thread's
+// share of them, eight 16-byte loads in flight at a time: one load at a time, a
+// workgroup with few waves waits out one memory latency per row.  Rows that are
+// not a multiple of 4 ids, or not 16-byte aligned, go by 4-byte loads.
+template <int NTHR, typename F>
+__device__ __forceinline__ void fta_each_id(const int32_t* __restrict__ p, int rows, int W, F f) {
+    constexpr int U = 8;
+    if ((W & 3) == 0 && ((uintptr_t)p & 15) == 0) {
+        const int w4 = W >> 2, n = rows * w4;
+        const int4* __restrict__ p4 = reinterpret_cast<const int4*>(p);
+        for (int e0 = threadIdx.x; e0 < n; e0 += U * NTHR) {
+            int4 v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                v[u] = (e0 + u * NTHR < n) ? p4[e0 + u * NTHR] : make_int4(-1, -1, -1, -1);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int r = (e0 + u * NTHR) / w4;
+                f(r, v[u].x);
+                f(r, v[u].y);
+                f(r, v[u].z);
+                f(r, v[u].w);
+            }
+        }
+    } else {
+        const int n = rows * W;
+        for (int e0 = threadIdx.x; e0 < n; e0 += U * NTHR) {
+            int v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = (e0 + u * NTHR < n) ? p[e0 + u * NTHR] : -1;
+#pragma unroll
+            for (int u = 0; u < U; ++u) f((e0 + u * NTHR) / W, v[u]);
+        }
+    }
+}
+
 // Membership bitmap sel[bh][m][qw]: bit (qm & 31) of word qw = qm / 32 is set
 // when q-block qm's merged list holds KV block m.  One workgroup per (bh, qw)
 // builds that word column for every m in LDS (atomicOr there), a chunk of
 // kSelChunk blocks at a time, and writes every word: no global atomics and no
-// separate clearing pass.
+// separate clearing pass.  The workgroups also form lse2 = lse * log2(e) (n_lse
+// values; the fp32 product that the dK/dV kernel would form per element) if lse is
+// set: it needs no launch of its own.  Latency-bound on small grids (8 workgroups at
+// N2048 H8 g64): 22 -> 8 us there with the loads of fta_each_id, 24 -> 16 us at
+// N32768 H32 g32.
 constexpr int kSelChunk = 8192;
 
 __global__ __launch_bounds__(256) void fta_sel_bitmap_kernel(const int32_t* __restrict__ merged, int QM, int W,
-                                                             int M, int QW, uint32_t* __restrict__ sel) {
+                                                             int M, int QW, uint32_t* __restrict__ sel,
+                                                             const float* __restrict__ lse, float* __restrict__ lse2,
+                                                             int64_t n_lse) {
     __shared__ uint32_t bits[kSelChunk];
     const int64_t bh = blockIdx.x / QW;
     const int qw = (int)(blockIdx.x - bh * QW);
     const int q0 = qw * 32, nq = min(32, QM - q0);
     const int32_t* mp = merged + (bh * QM + q0) * (int64_t)W;
+    if (lse != nullptr)
+        for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_lse; i += (int64_t)gridDim.x * 256)
+            lse2[i] = lse[i] * 1.4426950408889634f;
     for (int m0 = 0; m0 < M; m0 += kSelChunk) {
         const int mn = min(kSelChunk, M - m0);
         for (int i = threadIdx.x; i < mn; i += 256) bits[i] = 0u;
         __syncthreads();
-        for (int qq = 0; qq < nq; ++qq)
-            for (int e = threadIdx.x; e < W; e += 256) {
-                const int m = mp[(int64_t)qq * W + e] - m0;
-                if (m >= 0 && m < mn) atomicOr(&bits[m], 1u << qq);
-            }
+        fta_each_id<256>(mp, nq, W, [&](int qq, int id) {
+            const int m = id - m0;
+            if (m >= 0 && m < mn) atomicOr(&bits[m], 1u << qq);
+        });
         __syncthreads();
         for (int i = threadIdx.x; i < mn; i += 256) sel[(bh * M + m0 + i) * QW + qw] = bits[i];
         __syncthreads();
     }
 }
+
 
 // One wave per (bh, m): ascending q-block list, -1 fill, count.
 __global__ __launch_bounds__(64) void fta_reverse_lists_kernel(const uint32_t* __restrict__ sel, int QM, int QW,
@@ -672,39 +717,61 @@ __global__ __launch_bounds__(256) void fta_kv_order_kernel(const uint32_t* __res
     // head's whole bitmap: small heads rank in slices of 256 (the ranking, O(M)
     // per block, dominates), heads of more than 1024 blocks in slices of 1024
     // (four times fewer bitmap re-reads).
-    __shared__ uint32_t key[4096];
+    __shared__ __align__(16) uint32_t key[4096];
     __shared__ int s_work;
     const int64_t rk = blockIdx.x;               // (b, K/V head)
     const int slice = blockIdx.y;
     const int64_t bh = (rk / (H / G)) * H + (rk % (H / G)) * G;  // its first query head
     const uint32_t* rows = sel + bh * (int64_t)M * QW;
-    for (int m = threadIdx.x; m < M; m += 256) key[m] = 0xffffffffu;
+    const int M4 = (M + 3) & ~3;
+    for (int m = threadIdx.x; m < M4; m += 256) key[m] = 0u;
     if (threadIdx.x == 0) s_work = M;  // one setup step per block
     __syncthreads();
-    const int64_t nw = (int64_t)M * QW;
     int cw = 0;
-    for (int64_t i0 = threadIdx.x; i0 < nw; i0 += 8 * 256) {
-        uint32_t wv[8];  // eight loads in flight before any use
+    auto add = [&](int m, int c) {
+        if (c) atomicAdd(&key[m], (uint32_t)c);
+        cw += c;
+    };
+    if ((QW & 3) == 0 && ((uintptr_t)rows & 15) == 0) {  // eight 16-byte loads in flight
+        const int w4 = QW >> 2;
+        const int nw = M * w4;  // M <= 4096, QW words: below 2^31 for every QM the caller takes
+        const uint4* r4 = reinterpret_cast<const uint4*>(rows);
+        for (int i0 = threadIdx.x; i0 < nw; i0 += 8 * 256) {
+            uint4 wv[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) wv[u] = (i0 + u * 256 < nw) ? rows[i0 + u * 256] : 0u;
+            for (int u = 0; u < 8; ++u) wv[u] = (i0 + u * 256 < nw) ? r4[i0 + u * 256] : make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int c = __builtin_popcount(wv[u]);
-            if (c) atomicSub(&key[(i0 + u * 256) / QW], (uint32_t)c);
-            cw += c;
+            for (int u = 0; u < 8; ++u)
+                add(min((i0 + u * 256) / w4, M - 1), __builtin_popcount(wv[u].x) + __builtin_popcount(wv[u].y) +
+                                                         __builtin_popcount(wv[u].z) + __builtin_popcount(wv[u].w));
+        }
+    } else {
+        const int64_t nw = (int64_t)M * QW;
+        for (int64_t i0 = threadIdx.x; i0 < nw; i0 += 8 * 256) {
+            uint32_t wv[8];  // eight loads in flight before any use
+#pragma unroll
+            for (int u = 0; u < 8; ++u) wv[u] = (i0 + u * 256 < nw) ? rows[i0 + u * 256] : 0u;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int64_t m = (i0 + u * 256) / QW;
+                add(m < M ? (int)m : M - 1, __builtin_popcount(wv[u]));
+            }
         }
     }
     atomicAdd(&s_work, cw);
     __syncthreads();
     if (slice == 0 && threadIdx.x == 0) head_work[rk] = s_work;
+    // rank = blocks with a larger count, or the same count and a lower id; four keys per
+    // LDS read (the entries past M hold 0 and are never before a block with i < M)
     for (int u = 0; u < slice_blocks / 256; ++u) {
         const int i = slice * slice_blocks + u * 256 + threadIdx.x;
         if (i < M) {
             const uint32_t ki = key[i];
             int rank = 0;
-            for (int j = 0; j < M; ++j) {
-                const uint32_t kj = key[j];
-                rank += (kj < ki) || (kj == ki && j < i);
+            for (int j = 0; j < M4; j += 4) {
+                const uint4 k = *reinterpret_cast<const uint4*>(&key[j]);
+                rank += (k.x > ki || (k.x == ki && j < i)) + (k.y > ki || (k.y == ki && j + 1 < i)) +
+                        (k.z > ki || (k.z == ki && j + 2 < i)) + (k.w > ki || (k.w == ki && j + 3 < i));
             }
             order[rk * M + rank] = i;
         }
@@ -720,6 +787,14 @@ __global__ __launch_bounds__(256) void fta_kv_order_kernel(const uint32_t* __res
 // n not a multiple of 8, or above 4096 heads: identity.
 // With `part` set, each head's work is first formed from its partial counts:
 // head_work[i] = base + scale * sum_j part[i][j] (j < nparts).
+// The 64-bit value of the lane that DPP control CTRL names (within a row of 16).
+template <int CTRL>
+__device__ __forceinline__ long long fta_dpp64(long long x) {
+    const int lo = __builtin_amdgcn_mov_dpp((int)x, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(x >> 32), CTRL, 0xf, 0xf, true);
+    return ((long long)hi << 32) | (uint32_t)lo;
+}
+
 __global__ __launch_bounds__(256) void fta_head_balance_kernel(int32_t* __restrict__ head_work,
                                                                const int32_t* __restrict__ part, int nparts,
                                                                int base, int scale, int n,
@@ -727,10 +802,21 @@ __global__ __launch_bounds__(256) void fta_head_balance_kernel(int32_t* __restri
     __shared__ int w[4096];
     __shared__ int by_rank[4096];
     if (part != nullptr) {
-        for (int i = threadIdx.x; i < n; i += 256) {
-            int c = 0;
-            for (int j = 0; j < nparts; ++j) c += part[(int64_t)i * nparts + j];
-            head_work[i] = base + scale * c;
+        // head_work[i] = base + scale * sum of its parts: a wave takes eight heads at a
+        // time, their loads in flight together
+        const int lane = threadIdx.x & 63;
+        for (int i0 = (threadIdx.x >> 6) * 8; i0 < n; i0 += 32) {
+            int c[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+            for (int j = lane; j < nparts; j += 64)
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (i0 + u < n) c[u] += part[(int64_t)(i0 + u) * nparts + j];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+#pragma unroll
+                for (int off = 32; off > 0; off >>= 1) c[u] += __shfl_xor(c[u], off, 64);
+                if (lane == 0 && i0 + u < n) head_work[i0 + u] = base + scale * c[u];
+            }
         }
         __syncthreads();
     }
@@ -747,27 +833,29 @@ __global__ __launch_bounds__(256) void fta_head_balance_kernel(int32_t* __restri
         by_rank[rank] = i;
     }
     __syncthreads();
-    // greedy placement by the first wave: lane x < 8 keeps bin x's load and fill
+    // greedy placement by the first wave: lane x < 8 keeps bin x's load and fill (the
+    // least load by DPP: a shuffle through LDS cost three round trips per head)
     if (threadIdx.x < 64) {
         const int x = threadIdx.x;
         const int cap = n / 8;
         long long load = 0;
         int fill = 0;
+        int hd = by_rank[0];
         for (int r = 0; r < n; ++r) {
-            const int hd = by_rank[r];
+            const int next = by_rank[min(r + 1, n - 1)];  // read ahead of the reduction
+            const int wh = w[hd];
             // the open bin with the least load (ties: lowest bin)
             long long key = (x < 8 && fill < cap) ? load * 8 + x : 0x7fffffffffffffffll;
-#pragma unroll
-            for (int off = 4; off > 0; off >>= 1) {
-                const long long o = __shfl_xor(key, off, 8);
-                key = o < key ? o : key;
-            }
+            key = min(key, fta_dpp64<0xB1>(key));   // lane ^ 1
+            key = min(key, fta_dpp64<0x4E>(key));   // lane ^ 2
+            key = min(key, fta_dpp64<0x141>(key));  // 7 - lane: the other four
             const int best = (int)(key & 7);
             if (x == best) {
                 perm[best * cap + fill] = hd;
                 ++fill;
-                load += w[hd];
+                load += wh;
             }
+            hd = next;
         }
     }
 }
@@ -796,12 +884,11 @@ __global__ __launch_bounds__(256) void fta_head_work_union_kernel(const int32_t*
         if (tid == 0) s_u = 0;
         __syncthreads();
         const int q0 = gi * qpg, q1 = min(QM, q0 + qpg);
-        const int32_t* rows = merged + ((int64_t)bh * QM + q0) * W;
-        const int n = (q1 - q0) * W;
-        for (int e = tid; e < n; e += 256) {
-            const int m = rows[e];
-            if (m >= 0 && m < M) atomicOr(&bits[m >> 5], 1u << (m & 31));
-        }
+        fta_each_id<256>(merged + ((int64_t)bh * QM + q0) * W, q1 - q0, W, [&](int, int m) {
+            // most ids repeat: a read first keeps the atomics (which serialise on the few
+            // words of a short sequence) to the ids seen first
+            if (m >= 0 && m < M && !((bits[m >> 5] >> (m & 31)) & 1u)) atomicOr(&bits[m >> 5], 1u << (m & 31));
+        });
         __syncthreads();
         int c = (tid < 128) ? __popc(bits[tid]) : 0;
         for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
@@ -950,11 +1037,12 @@ __global__ __launch_bounds__(256) void fta_qblock_union_kernel(const int32_t* __
 
 namespace fta {
 
-int launch_sel_bitmap(const int32_t* merged, int BH, int QM, int W, int M, uint32_t* sel, hipStream_t st) {
+int launch_sel_bitmap(const int32_t* merged, int BH, int QM, int W, int M, uint32_t* sel, const float* lse,
+                      float* lse2, int64_t n_lse, hipStream_t st) {
     const int QW = (QM + 31) / 32;
     if ((int64_t)BH * QW == 0 || M <= 0) return FTA_OK;
     hipLaunchKernelGGL(fta_sel_bitmap_kernel, dim3((unsigned)((int64_t)BH * QW)), dim3(256), 0, st, merged, QM, W,
-                       M, QW, sel);
+                       M, QW, sel, lse, lse2, n_lse);
     return check_launch("fta_sel_bitmap_kernel");
 }
 
@@ -1111,7 +1199,7 @@ int fta_build_reverse_indices(const int32_t* merged_indices, const int32_t* coun
         return fta::arg_error("build_reverse_indices: workspace too small");
     hipStream_t st = (hipStream_t)stream;
     uint32_t* sel = (uint32_t*)workspace;
-    int rc = fta::launch_sel_bitmap(merged_indices, B * H, QM, W, M, sel, st);
+    int rc = fta::launch_sel_bitmap(merged_indices, B * H, QM, W, M, sel, nullptr, nullptr, 0, st);
     if (rc != FTA_OK) return rc;
     const int QW = (QM + 31) / 32;
     hipLaunchKernelGGL(fta_reverse_lists_kernel, dim3((unsigned)((int64_t)B * H * M)), dim3(64), 0, st, sel, QM, QW,

@@ -64,3 +64,27 @@ def test_wide_token_strides(D, b):
         x, y = x.float().cpu().numpy(), y.float().cpu().numpy()
         step = np.maximum(np.abs(x), np.abs(y)) * 2.0**-7 + np.abs(x).max() * 2.0**-16
         assert (np.abs(x - y) <= step).all(), name
+
+
+@pytest.mark.parametrize("W,offset", [(5, 0), (8, 0), (8, 1), (12, 2), (1, 3)])
+def test_list_loads(W, offset):
+    """Merged lists are read 16 bytes at a time where a row is a multiple of 4 ids on a
+    16-byte boundary, 4 bytes otherwise: the same lists in any width and at any
+    alignment (padded with -1, or at an odd place in a buffer) give the same bits."""
+    B, H, N, D, g, b = 1, 2, 700, 64, 16, 64
+    say(f"[list loads] W{W} offset {offset}")
+    qpad, kvpad = (0, 4), (0, 4)
+    merged = torch.from_numpy(_random_merged(B, H, 44, W, 11, 5)).cuda()
+    base = torch.full((B, H, 44, 16), -1, dtype=torch.int32, device="cuda")
+    base[..., :W] = merged
+    buf = torch.empty(merged.numel() + offset, dtype=torch.int32, device="cuda")
+    placed = buf[offset:].view(merged.shape).copy_(merged)
+    assert placed.is_contiguous() and placed.data_ptr() % 16 == 4 * offset
+    q, k, v, do = (rand((B, N, H * D), 50 + i, torch.bfloat16, "cuda") for i in range(4))
+    res = []
+    for lists in (base, placed):
+        ql, kl, vl = (x.detach().requires_grad_(True) for x in (q, k, v))
+        o, lse = fta.flash_topk_attn(ql, kl, vl, lists, None, H, g, b, None, None, kvpad, qpad)
+        res.append([o.detach(), lse, *torch.autograd.grad(o, (ql, kl, vl), do)])
+    for x, y in zip(*res):
+        assert torch.equal(x, y)
