@@ -496,11 +496,14 @@ __global__ __launch_bounds__(256 * (2 / QT), (D > 160) ? 1 : 2) void fta_block_s
 //    per SIMD;
 //  * the rare exact path recomputes block m's scores from its LDS buffer.
 // ----------------------------------------------------------------------------
-template <int D>
+// BK: keys of a chunk that are used, 64 or 48 (b = 48: one block per chunk; the rows
+// past its keys are not gathered where whole instructions allow, and never read back).
+template <int D, int BK>
 struct ScorePipeShape {
     static constexpr int QSEG = D / 8;
     static constexpr int SLOTS = 64 * QSEG;  // 16-byte slots per K block
-    static constexpr int LQ = SLOTS / 256;   // DMA instructions per wave per block (4 waves)
+    static constexpr int LQ = (BK * QSEG + 255) / 256;  // DMA instructions per wave per block (4 waves)
+    static constexpr int ROWS = LQ * 256 / QSEG;        // rows they gather
     static constexpr int NBUF = 4;
     static constexpr int BUF_B = SLOTS * 16;
     static_assert(SLOTS % 256 == 0, "whole DMA instructions per wave");
@@ -592,7 +595,14 @@ __device__ __forceinline__ uint32_t fta_f2h2(float lo, float hi) {
 // formed at its last chunk from the chunk totals, all taken against the row's
 // running reference R (an exact-path re-reference inside a block rescales the
 // block's earlier chunks, as it rescales the row total).
-template <int DT, int D, int NG, int GT = 2, bool GH = false, int SB = 1>
+// BK = 48 (b = 48, SB = 1): a chunk is one block of 48 keys.  Its second half's
+// scores are 16 keys, registers 0 .. 7 of each lane in the 32 x 32 layout, so only
+// those eight exponentials are formed; the products of the 16 rows past them are
+// wasted (a quarter of the MFMAs) and their results dropped.  The values are those of
+// the unpipelined kernel bit for bit (its masked terms add exact zeros).  B1 N4032 H32
+// D128 top-16: scoring kernel 0.328 -> 0.183 ms, with streams in place of per-block
+// values (selector 0.078 -> 0.059 ms).
+template <int DT, int D, int NG, int GT = 2, bool GH = false, int SB = 1, int BK = 64>
 __device__ __forceinline__ void fta_score_tile(const ScoreArgs& a, const int wg) {
     const uint16_t* __restrict__ q = a.q;
     const uint16_t* __restrict__ k = a.k;
@@ -603,14 +613,16 @@ __device__ __forceinline__ void fta_score_tile(const ScoreArgs& a, const int wg)
     // NG > 0: candidate streams with NG block groups (STREAM)
     constexpr bool STREAM = NG > 0;
     using E = Elem<DT>;
-    using Sh = ScorePipeShape<D>;
+    using Sh = ScorePipeShape<D, BK>;
     using SW = FtaSwz<Sh::QSEG>;
     constexpr int KS = D / 16;
     constexpr int QSEG = Sh::QSEG, LQ = Sh::LQ, NBUF = Sh::NBUF;
     __shared__ __align__(1024) unsigned char sK[NBUF][Sh::BUF_B];
     static_assert(GT == 2 || GT == 4, "group top-2 or top-4");
     static_assert(!GH || GT == 4, "fp16 group state holds four keys");
-    static_assert(SB == 1 || SB == 2, "blocks of 64 or 128 keys");
+    static_assert(SB == 1 || (SB == 2 && BK == 64), "blocks of 48, 64 or 128 keys");
+    static_assert(BK == 64 || BK == 48, "16-key granules of a chunk's second half");
+    constexpr int NE1 = (BK - 32) / 2;  // scores per lane and query tile of a chunk's second half
     constexpr int GB = GT * (GH ? 2 : 4);  // bytes per (group, query)
     using GRaw = typename GroupRaw<GB>::type;
     __shared__ __align__(16) GRaw sG[STREAM ? NG : 1][256];
@@ -654,8 +666,8 @@ __device__ __forceinline__ void fta_score_tile(const ScoreArgs& a, const int wg)
     const int U = M * SB;  // 64-key chunks
     auto issue = [&](int u) {
         const uint32_t sb = lds0 + (u & (NBUF - 1)) * Sh::BUF_B;
-        const int kb = u * 64 - pad_head;
-        if (kb >= 0 && kb + 64 <= N) {
+        const int kb = u * BK - pad_head;
+        if (kb >= 0 && kb + Sh::ROWS <= N) {
             const uint16_t* base = kp + (int64_t)kb * k_sn;
 #pragma unroll
             for (int i = 0; i < LQ; ++i) fta_dma16_so(base, roff[i], sb + (i * 4 + wave) * 1024);
@@ -688,8 +700,8 @@ __device__ __forceinline__ void fta_score_tile(const ScoreArgs& a, const int wg)
         }
     };
     auto edge_mask = [&](int u, int s, f32x16 (&acc)[2]) {
-        const int kb = u * 64 - pad_head;
-        if (kb < 0 || kb + 64 > N) {
+        const int kb = u * BK - pad_head;
+        if (kb < 0 || kb + BK > N) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const int t = kb + s * 32 + c_row(i, lane);
@@ -700,35 +712,40 @@ __device__ __forceinline__ void fta_score_tile(const ScoreArgs& a, const int wg)
             }
         }
     };
-    auto sums16 = [&](const f32x16 (&acc)[2], const float* Rr, float* e) {
+    // sums of the first `ne` scores of a half (16, or NE1 in the second half)
+    auto sums = [&](const f32x16 (&acc)[2], const float* Rr, float* e, auto ne) {
+        constexpr int NE = decltype(ne)::value;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            float v[16];
+            float v[NE];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = acc[t][i];
-            e[t] = fta_sum_exp2<16>(v, c, Rr[t]);
+            for (int i = 0; i < NE; ++i) v[i] = acc[t][i];
+            e[t] = fta_sum_exp2<NE>(v, c, Rr[t]);
         }
     };
+    using E16 = std::integral_constant<int, 16>;
+    using EH1 = std::integral_constant<int, NE1>;
     // R[t]: reference of tile t's query (lane & 31), used by this lane's exps of both
     // tiles; L: running total of the lane's own (tile lane >> 5, query lane & 31)
     float R[2] = {-FTA_INF, -FTA_INF}, L = 0.f;
     const bool own1 = lane >= 32;
     float Rown = -FTA_INF;  // R of the lane's own tile (R[lane >> 5])
     // One pipeline stage, written in issue order: the MFMAs of half s of block mb
-    // (into dst) interleaved with the exps of src, 32 / KS exps after each MFMA
-    // pair.  The sums use the same 16-term tree as fta_sum_exp2<16>.
+    // (into dst) interleaved with the exps of src's first NE scores per tile, 2 NE / KS
+    // exps after each MFMA pair.  The sums use the same tree as fta_sum_exp2<NE>.
     // The order is pinned with empty volatile asm statements (kept in program
     // order by the compiler): group g's K fragment and a scalar copy of the
     // scale used by its exps pass through one, and its exp / add results feed
     // the next group's, so each group's MFMAs, exps and adds stay in their window.
-    auto stage = [&](int bi, int s, f32x16 (&dst)[2], const f32x16 (&src)[2], float* e_out) {
+    auto stage = [&](int bi, int s, f32x16 (&dst)[2], const f32x16 (&src)[2], float* e_out, auto ne) {
+        constexpr int NE = decltype(ne)::value;
         const uint16_t* base = reinterpret_cast<const uint16_t*>(&sK[bi][0]) + s * 32 * QSEG * 8;
         const f32x16 zacc = {};
         uint4 a[KS];
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) a[ks] = *reinterpret_cast<const uint4*>(base + SW::off(lane & 31, 2 * ks + hf));
-        constexpr int PER = 32 / KS;
-        float ex[2][16];
+        constexpr int PER = 2 * NE / KS;
+        float ex[2][NE];
 #pragma unroll
         for (int g = 0; g < KS; ++g) {
             typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
@@ -740,7 +757,7 @@ __device__ __forceinline__ void fta_score_tile(const ScoreArgs& a, const int wg)
             dst[1] = E::mma(ag, qf[1][g], g ? dst[1] : zacc);
 #pragma unroll
             for (int u = 0; u < PER; ++u) {
-                const int idx = g * PER + u, t = idx >> 4, i = idx & 15;
+                const int idx = g * PER + u, t = idx / NE, i = idx % NE;
                 ex[t][i] = fta_exp2(fmaf(src[t][i], cg, -R[t]));
             }
             // tree adds whose subtree is complete after this group (same tree and
@@ -748,16 +765,16 @@ __device__ __forceinline__ void fta_score_tile(const ScoreArgs& a, const int wg)
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int w = 1; w < 16; w <<= 1)
+                for (int w = 1; w < NE; w <<= 1)
 #pragma unroll
-                    for (int i = 0; i + w < 16; i += 2 * w)
-                        if ((t * 16 + i + 2 * w - 1) / PER == g) {
+                    for (int i = 0; i + w < NE; i += 2 * w)
+                        if ((t * NE + i + 2 * w - 1) / PER == g) {
                             ex[t][i] += ex[t][i + w];
                             asm volatile("" ::"v"(ex[t][i]));
                         }
 #pragma unroll
             for (int u = 0; u < PER; ++u) {
-                const int idx = g * PER + u, t = idx >> 4, i = idx & 15;
+                const int idx = g * PER + u, t = idx / NE, i = idx % NE;
                 if (i & 1) asm volatile("" ::"v"(ex[t][i]));  // odd leaves are consumed by level-1 adds
             }
         }
@@ -879,7 +896,7 @@ __device__ __forceinline__ void fta_score_tile(const ScoreArgs& a, const int wg)
             if (blast) gtop = sG[gslot][tid];
 
         float e0[2], e1[2];
-        const int kb = u * 64 - pad_head;
+        const int kb = u * BK - pad_head;
         if (IN || u + 1 < U) {
             // Every block but the last runs the same two stages; a block at a
             // sequence edge first masks its scores in place (uniform branches),
@@ -887,20 +904,20 @@ __device__ __forceinline__ void fta_score_tile(const ScoreArgs& a, const int wg)
             // their registers.  Masked scores are -inf: their exps are 0.
             // pad_head, pad_tail < b and b | pad_head + N + pad_tail (checked on the host):
             // only the chunks of the first and the last block can reach past the sequence
-            const bool edge = !IN && (kb < 0 || kb + 64 > N);
+            const bool edge = !IN && (kb < 0 || kb + BK > N);
             if (edge) edge_mask(u, 0, h0);
-            stage(bm, 1, h1, h0, e0);     // MFMAs of half 1 of chunk u, exps of half 0
+            stage(bm, 1, h1, h0, e0, E16{});     // MFMAs of half 1 of chunk u, exps of half 0
             if (edge) edge_mask(u, 1, h1);
-            stage(bn, 0, h0, h1, e1);     // MFMAs of half 0 of chunk u + 1, exps of half 1
+            stage(bn, 0, h0, h1, e1, EH1{});     // MFMAs of half 0 of chunk u + 1, exps of half 1
         } else {
             edge_mask(u, 0, h0);
             mma_half(bm, 1, h1);
-            sums16(h0, R, e0);
+            sums(h0, R, e0, E16{});
             edge_mask(u, 1, h1);
             if (u + 1 < U) {
                 mma_half(bn, 0, h0);
             }
-            sums16(h1, R, e1);
+            sums(h1, R, e1, EH1{});
         }
         // chunk total of the lane's own (tile, query): lanes l and l ^ 32 hold halves
         // of each query's sum; one lane-half swap adds them (the same operand pairs as
@@ -931,7 +948,7 @@ __device__ __forceinline__ void fta_score_tile(const ScoreArgs& a, const int wg)
 #pragma unroll
                     for (int i = 1; i < 16; ++i) mx = fmaxf(mx, x0[t][i]);
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, x1[t][i]);
+                    for (int i = 0; i < NE1; ++i) mx = fmaxf(mx, x1[t][i]);
                     mx = fmaxf(mx, fta_xor32(mx));
                     R[t] = (mx == -FTA_INF) ? 0.f : mx * c;
                 }
@@ -940,8 +957,8 @@ __device__ __forceinline__ void fta_score_tile(const ScoreArgs& a, const int wg)
                 L = (L > 0.f) ? L * fta_exp2(R_old - R_new) : 0.f;
                 if constexpr (SB > 1) bsum = (bsum > 0.f) ? bsum * fta_exp2(R_old - R_new) : 0.f;
                 float f0[2], f1[2];
-                sums16(x0, R, f0);
-                sums16(x1, R, f1);
+                sums(x0, R, f0, E16{});
+                sums(x1, R, f1, EH1{});
                 float tot[2];
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
@@ -1137,9 +1154,9 @@ __device__ __forceinline__ void fta_score_tile(const ScoreArgs& a, const int wg)
     }
 }
 
-template <int DT, int D, int NG, int GT, bool GH, int SB>
+template <int DT, int D, int NG, int GT, bool GH, int SB, int BK>
 __global__ __launch_bounds__(256, 2) void fta_block_score_lse_pipe_kernel(const ScoreArgs a) {
-    fta_score_tile<DT, D, NG, GT, GH, SB>(a, fta_xcd_remap(blockIdx.x, a.total));
+    fta_score_tile<DT, D, NG, GT, GH, SB, BK>(a, fta_xcd_remap(blockIdx.x, a.total));
 }
 
 // ----------------------------------------------------------------------------
@@ -1765,7 +1782,7 @@ __global__ void fta_stream_reset_kernel(int* __restrict__ ctrs) {
 // top-k from the slot with the selector of the per-block-value path.  The
 // results equal the stream path's (both selectors are exact); only the time
 // differs.
-template <int DT, int D, int KB, int SB>
+template <int DT, int D, int KB, int SB, int BK>
 __global__ __launch_bounds__(256, 1) void fta_stream_fallback_kernel(ScoreArgs a, const int* __restrict__ ovf_list,
                                                                     const int* __restrict__ ovf_cnt,
                                                                     float* __restrict__ slots, int m_out,
@@ -1783,7 +1800,7 @@ __global__ __launch_bounds__(256, 1) void fta_stream_fallback_kernel(ScoreArgs a
     for (int r = blockIdx.x; r < n; r += gridDim.x) {
         const int tile = __builtin_amdgcn_readfirstlane(ovf_list[r]);
         if ((unsigned)tile >= (unsigned)a.total) continue;  // workgroup-uniform
-        fta_score_tile<DT, D, 0, 2, false, SB>(a, tile);
+        fta_score_tile<DT, D, 0, 2, false, SB, BK>(a, tile);
         __syncthreads();  // the slot is complete
         const int bh = tile / a.qtiles, qt = tile - bh * a.qtiles;
         const int64_t r0 = (int64_t)bh * a.N + qt * 256;
@@ -1884,11 +1901,11 @@ __global__ __launch_bounds__(256) void fta_topk_select_sort_kernel(
 
 namespace {
 
-// The pipelined scoring kernel serves b = 64 and b = 128 with D <= 128 (run as 64
+// The pipelined scoring kernel serves b = 48, 64 and 128 with D <= 128 (run as 64
 // or 128 columns, the columns past D multiplied by zero q columns) and a K token
 // stride whose 64-row offsets fit 32 bits.
 bool score_pipe_ok(int bsz, int Dk, const int64_t* ks) {
-    return (bsz == 64 || bsz == 128) && Dk <= 128 && ks[2] >= 0 && ks[2] <= (1 << 24);
+    return (bsz == 48 || bsz == 64 || bsz == 128) && Dk <= 128 && ks[2] >= 0 && ks[2] <= (1 << 24);
 }
 
 // Candidate streams of the pipelined kernel (STREAM = true), laid out in the
@@ -1968,15 +1985,17 @@ int launch_score_lse_dt(const void* q, const void* k, int B, int H, int N, int D
     }
     const ScoreArgs sa = score_args(q, k, B, H, N, D, qs, ks, M, bsz, pad_head, pad_tail, scale, blk_lse, row_lse,
                                     kgroups, tau, sb);
-#define FTA_LAUNCH_PIPE_SB(DK, NG, GT, GH, SB)                                                             \
-    hipLaunchKernelGGL((fta_block_score_lse_pipe_kernel<DT, (DK <= 64) ? 64 : 128, NG, GT, GH, SB>),        \
+#define FTA_LAUNCH_PIPE_SB(DK, NG, GT, GH, SB, BK)                                                         \
+    hipLaunchKernelGGL((fta_block_score_lse_pipe_kernel<DT, (DK <= 64) ? 64 : 128, NG, GT, GH, SB, BK>),    \
                        dim3(total), dim3(256), 0, st, sa)
 #define FTA_LAUNCH_PIPE(DK, NG, GT, GH)                                                                    \
     do {                                                                                                   \
         if (bsz == 64)                                                                                     \
-            FTA_LAUNCH_PIPE_SB(DK, NG, GT, GH, 1);                                                         \
+            FTA_LAUNCH_PIPE_SB(DK, NG, GT, GH, 1, 64);                                                     \
+        else if (bsz == 48)                                                                                \
+            FTA_LAUNCH_PIPE_SB(DK, NG, GT, GH, 1, 48);                                                     \
         else                                                                                               \
-            FTA_LAUNCH_PIPE_SB(DK, NG, GT, GH, 2);                                                         \
+            FTA_LAUNCH_PIPE_SB(DK, NG, GT, GH, 2, 64);                                                     \
     } while (0)
 #define FTA_LAUNCH_SCORE(DK)                                                                               \
     if (pipe && sb.pool != nullptr && sb.m_out <= 8)                                                       \
@@ -2255,17 +2274,21 @@ int launch_stream_select_dt(const ScoreArgs& sa, int Dk, const StreamBufs& sb, i
     int rc = fta::check_launch("fta_topk_stream_kernel");
     if (rc != FTA_OK) return rc;
     const int grid = sa.total < kStreamSlots ? sa.total : kStreamSlots;
-#define FTA_LAUNCH_FALLBACK(DK, SB)                                                                             \
-    hipLaunchKernelGGL((fta_stream_fallback_kernel<DT, DK, 32, SB>), dim3(grid), dim3(256), 0, s, sa, sb.ovf_list, \
-                       sb.ctrs + 1, sb.slots, m_out, threshold, idx, raw, avg)
+#define FTA_LAUNCH_FALLBACK(DK, SB, BK)                                                                         \
+    hipLaunchKernelGGL((fta_stream_fallback_kernel<DT, DK, 32, SB, BK>), dim3(grid), dim3(256), 0, s, sa,         \
+                       sb.ovf_list, sb.ctrs + 1, sb.slots, m_out, threshold, idx, raw, avg)
     if (Dk <= 64 && sa.bsz == 64)
-        FTA_LAUNCH_FALLBACK(64, 1);
+        FTA_LAUNCH_FALLBACK(64, 1, 64);
+    else if (Dk <= 64 && sa.bsz == 48)
+        FTA_LAUNCH_FALLBACK(64, 1, 48);
     else if (Dk <= 64)
-        FTA_LAUNCH_FALLBACK(64, 2);
+        FTA_LAUNCH_FALLBACK(64, 2, 64);
     else if (sa.bsz == 64)
-        FTA_LAUNCH_FALLBACK(128, 1);
+        FTA_LAUNCH_FALLBACK(128, 1, 64);
+    else if (sa.bsz == 48)
+        FTA_LAUNCH_FALLBACK(128, 1, 48);
     else
-        FTA_LAUNCH_FALLBACK(128, 2);
+        FTA_LAUNCH_FALLBACK(128, 2, 64);
 #undef FTA_LAUNCH_FALLBACK
     return fta::check_launch("fta_stream_fallback_kernel");
 }
@@ -2280,6 +2303,9 @@ int topk_score_checks(int B, int H, int N, int D, int bsz, int pad_head, int pad
     if (max_topk < 0) return fta::arg_error("topk_score: max_topk must be >= 0");
     *m_out = (max_topk > 0 && max_topk < *M) ? max_topk : *M;
     *streams = *m_out <= kStreamMaxTopk && score_pipe_ok(bsz, fta::kernel_head_dim(D), k_strides);
+    // b = 48 also takes the per-block-value path, in a workspace that holds only that
+    // (callers that sized it so before these blocks had streams)
+    if (bsz == 48 && *streams && workspace_bytes < stream_min_bytes(B, H, N, *M)) *streams = false;
     const size_t need = *streams ? stream_min_bytes(B, H, N, *M) : full_bytes(B, H, N, *M);
     if (workspace_bytes < need)
         return fta::arg_error("topk_score: workspace too small (see fta_topk_score_workspace_size_ex)");
@@ -2315,7 +2341,7 @@ int fta_topk_score_candidates(const void* q, const void* k, int dtype, int B, in
     int st = topk_score_checks(B, H, N, D, score_block_size, pad_head, pad_tail, max_topk, k_strides,
                                workspace_bytes, &M, &m_out, &streams);
     if (st != FTA_OK) return st;
-    if (!streams)
+    if (!streams || score_block_size == 48)
         return fta::unsupported("topk_score_candidates: needs b = 64 or 128, D <= 128 and at most 32 blocks per query");
     float* row_lse = nullptr;
     const StreamBufs sb = stream_layout(workspace, workspace_bytes, B, H, N, M, m_out, &row_lse);
@@ -2335,7 +2361,7 @@ int fta_topk_select_candidates(const void* q, const void* k, int dtype, int B, i
     int st = topk_score_checks(B, H, N, D, score_block_size, pad_head, pad_tail, max_topk, k_strides,
                                workspace_bytes, &M, &m_out, &streams);
     if (st != FTA_OK) return st;
-    if (!streams)
+    if (!streams || score_block_size == 48)
         return fta::unsupported("topk_select_candidates: needs b = 64 or 128, D <= 128 and at most 32 blocks per query");
     if (!topk_indices || !topk_raw || !topk_avg) return fta::arg_error("topk_select_candidates: null pointer");
     return stream_select(q, k, dtype, B, H, N, D, q_strides, k_strides, score_block_size, pad_head, pad_tail, scale,
