@@ -66,8 +66,8 @@ def flash_topk_score(
     raw = torch.empty(B, H, N, m_out, device=dev, dtype=torch.float32)
     avg = torch.empty(B, H, N, m_out, device=dev, dtype=torch.float32)
     L = _lib.lib()
-    ws = _lib.workspace(L.fta_topk_score_workspace_size_ex(B, H, N, Dp, score_block_size, pad_head, pad_tail, topk),
-                        dev)
+    ws = _lib.workspace(
+        _lib.size_of("fta_topk_score_workspace_size_ex", B, H, N, Dp, score_block_size, pad_head, pad_tail, topk), dev)
     rc = L.fta_topk_score(
         _lib.ptr(qq), _lib.ptr(kk), _lib.dtype_code(qq.dtype), B, H, N, Dp, _lib.i64arr(qs), _lib.i64arr(ks),
         score_block_size, pad_head, pad_tail, float(D ** -0.5), topk, float(threshold),

@@ -108,12 +108,25 @@ def stream_ptr(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+@lru_cache(maxsize=1024)
+def size_of(name: str, *geometry: int) -> int:
+    """A ``*_workspace_size`` of the library: a pure function of the geometry, so
+    repeated calls of one shape skip the ctypes call."""
+    return int(getattr(lib(), name)(*geometry))
+
+
 def ptr(t) -> int:
     return 0 if t is None else t.data_ptr()
 
 
+@lru_cache(maxsize=1024)
+def _i64const(vals: tuple):
+    return (ctypes.c_int64 * len(vals))(*vals)
+
+
 def i64arr(vals: Sequence[int]):
-    return (ctypes.c_int64 * len(vals))(*[int(v) for v in vals])
+    """Constant int64 array (strides); equal values share one, which the library only reads."""
+    return _i64const(tuple(map(int, vals)))
 
 
 def dtype_code(dt: torch.dtype) -> int:
@@ -135,22 +148,14 @@ def token_view(x: torch.Tensor, layout: str, num_heads: int):
     layout "bnc": x is [B, N, H*D]; layout "bhnd": x is [B, H, N, D].
     """
 
-    def ok(t, strides):
-        return (
-            t.stride(-1) == 1
-            and t.data_ptr() % 16 == 0
-            and all(int(s) % 8 == 0 for s in strides)
-        )
+    def ok(t, s0, s1, s2):
+        return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and (s0 | s1 | s2) & 7 == 0
 
     if layout == "bnc":
         D = x.shape[2] // num_heads
-        strides = [x.stride(0), D, x.stride(1)]
-        if not ok(x, strides):
+        if not ok(x, x.stride(0), D, x.stride(1)):
             x = x.contiguous()
-            strides = [x.stride(0), D, x.stride(1)]
-        return x, strides
-    strides = [x.stride(0), x.stride(1), x.stride(2)]
-    if not ok(x, strides):
+        return x, (x.stride(0), D, x.stride(1))
+    if not ok(x, x.stride(0), x.stride(1), x.stride(2)):
         x = x.contiguous()
-        strides = [x.stride(0), x.stride(1), x.stride(2)]
-    return x, strides
+    return x, (x.stride(0), x.stride(1), x.stride(2))

@@ -30,12 +30,12 @@ def _sparse_attn_fwd(q, k, v, merged, H, g, kvb, scale, q_padding, kv_padding, H
     QM, W = merged.shape[2], merged.shape[3]
     L = _lib.lib()
     geo = (B, H, N, D, g, kvb, q_padding[0], q_padding[1], kv_padding[0], kv_padding[1])
-    ws = _lib.workspace(L.fta_sparse_attn_fwd_workspace_size(*geo), dev)
+    ws = _lib.workspace(_lib.size_of("fta_sparse_attn_fwd_workspace_size", *geo), dev)
     rc = L.fta_sparse_attn_fwd_gqa(
         _lib.ptr(qq), _lib.i64arr(qs), _lib.ptr(kk), _lib.i64arr(ks), _lib.ptr(vv), _lib.i64arr(vs),
         _lib.dtype_code(q.dtype), B, H, Hk, N, D, _lib.ptr(merged), QM, W, g, kvb,
         q_padding[0], q_padding[1], kv_padding[0], kv_padding[1], float(scale),
-        _lib.ptr(o), _lib.i64arr([N * C, D, C]), _lib.ptr(lse), _lib.ptr(ws), ws.numel(),
+        _lib.ptr(o), _lib.i64arr((N * C, D, C)), _lib.ptr(lse), _lib.ptr(ws), ws.numel(),
         _lib.stream_ptr(dev),
     )
     _lib.check(rc, "flash_sparse_attn")

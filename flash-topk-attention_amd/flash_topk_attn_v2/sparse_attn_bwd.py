@@ -110,7 +110,7 @@ def sparse_attn_bwd(
     gk = [N * Hk * D, D, Hk * D]
     L = _lib.lib()
     geo = (B, H, N, D, q_block_size, kv_block_size, q_padding[0], q_padding[1], kv_padding[0], kv_padding[1])
-    ws = _lib.workspace(L.fta_sparse_attn_bwd_workspace_size(*geo), dev)
+    ws = _lib.workspace(_lib.size_of("fta_sparse_attn_bwd_workspace_size", *geo), dev)
     rc = L.fta_sparse_attn_bwd_gqa(
         _lib.ptr(qq), _lib.i64arr(qs), _lib.ptr(kk), _lib.i64arr(ks), _lib.ptr(vv), _lib.i64arr(vs),
         _lib.ptr(dd), _lib.i64arr(dos), _lib.dtype_code(q.dtype), B, H, Hk, N, D, _lib.ptr(merged), QM, W,
