@@ -178,7 +178,7 @@ __device__ int fta_build_q_masks(const AttnArgs& a, int bh, int p0, int seg0, in
 // lazily rescaled running max (rescale only when the max grows by > 2^8),
 // O^T += V^T P^T.
 // ----------------------------------------------------------------------------
-template <int DT, int D, int TPW, int NW>
+template <int DT, int D, int TPW, int NW, bool SPLIT>
 __global__ __launch_bounds__(NW * 64, 1) void fta_sparse_fwd_kernel(AttnArgs a) {
     using E = Elem<DT>;
     constexpr int NTHR = NW * 64;
@@ -195,8 +195,17 @@ __global__ __launch_bounds__(NW * 64, 1) void fta_sparse_fwd_kernel(AttnArgs a) 
     __shared__ int s_tmp[8];
 
     const int wgi = fta_xcd_remap(blockIdx.x, a.total);
-    const int bh = wgi / a.wg_per_bh;
-    const int wq = wgi - bh * a.wg_per_bh;
+    int bh, wq, sp = 0;  // (b, h), tile group, part (as in fta_sparse_fwd_pipe_kernel)
+    if constexpr (SPLIT) {
+        const int per = a.wg_per_bh * a.nsplit;
+        bh = wgi / per;
+        const int r = wgi - bh * per;
+        wq = r / a.nsplit;
+        sp = r - wq * a.nsplit;
+    } else {
+        bh = wgi / a.wg_per_bh;
+        wq = wgi - bh * a.wg_per_bh;
+    }
     const int b = bh / a.H, h = bh - (bh / a.H) * a.H;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int hf = lane >> 5;
@@ -239,12 +248,18 @@ __global__ __launch_bounds__(NW * 64, 1) void fta_sparse_fwd_kernel(AttnArgs a) 
     for (int seg0 = 0; seg0 < a.Mkv; seg0 += kSeg) {
         const int segn = min(kSeg, a.Mkv - seg0);
         const int U = fta_build_q_masks<T>(a, bh, p0, seg0, segn, sMask, sList, s_tmp);
-        if (U == 0) continue;
-        const int iters = U * nch;
+        int u_lo = 0, u_n = U;  // this part's union positions (workgroup-uniform)
+        if constexpr (SPLIT) {
+            u_lo = (U * sp) / a.nsplit;
+            u_n = (U * (sp + 1)) / a.nsplit - u_lo;
+        }
+        // no wave reads sMask / sList below when the part is empty
+        if (u_n == 0) continue;
+        const int iters = u_n * nch;
 
         auto load = [&](int it) {
             const int u = it / nch, ch = it - (it / nch) * nch;
-            const int m = seg0 + sList[u];
+            const int m = seg0 + sList[u_lo + u];
             const int kb = m * a.kvb - a.kv_pad + ch * 64;
             const int rem = a.kvb - ch * 64;
 #pragma unroll
@@ -276,7 +291,7 @@ __global__ __launch_bounds__(NW * 64, 1) void fta_sparse_fwd_kernel(AttnArgs a) 
             const int buf = it & 1;
             if (it + 1 < iters) load(it + 1);
             const int u = it / nch, ch = it - (it / nch) * nch;
-            const int ml = sList[u];
+            const int ml = sList[u_lo + u];
             const int m = seg0 + ml;
             const int kb = m * a.kvb - a.kv_pad + ch * 64;
             const int rem = a.kvb - ch * 64;
@@ -374,6 +389,21 @@ __global__ __launch_bounds__(NW * 64, 1) void fta_sparse_fwd_kernel(AttnArgs a) 
 #pragma unroll
     for (int tt = 0; tt < TPW; ++tt) {
         const float L = l_run[tt] + fta_xor32(l_run[tt]);
+        if constexpr (SPLIT) {
+            // the part's unnormalised O, its running max and sum, by padded position
+            const int p = p0 + 32 * (wave * TPW + tt) + (lane & 31);
+            if (p >= a.npq) continue;
+            const int64_t row = ((int64_t)sp * a.nbh + bh) * a.npq + p;
+            if (lane < 32) a.part_ml[row] = make_float2(m_run[tt], L);
+            float* po = a.part_o + row * D;
+#pragma unroll
+            for (int dt = 0; dt < DT32; ++dt)
+#pragma unroll
+                for (int i = 0; i < 16; i += 4)
+                    *reinterpret_cast<float4*>(po + dt * 32 + c_row(i, lane)) =
+                        make_float4(oacc[tt][dt][i], oacc[tt][dt][i + 1], oacc[tt][dt][i + 2], oacc[tt][dt][i + 3]);
+            continue;
+        }
         const float inv = (L > 0.f) ? 1.f / L : 0.f;
         const int t = p0 + 32 * (wave * TPW + tt) + (lane & 31) - a.q_pad;
         if (t < 0 || t >= a.N) continue;
@@ -2235,7 +2265,14 @@ int launch_fwd_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
     switch (Dk) {
 #define FTA_FWD(DK, TPW, NW)                                                                              \
     case DK:                                                                                              \
-        hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, DK, TPW, NW>), dim3(grid), dim3(NW * 64), 0, st, a); \
+        hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, DK, TPW, NW, false>), dim3(grid), dim3(NW * 64), 0, st, a); \
+        break;
+#define FTA_FWD_WIDE(DK, NW)                                                                              \
+    case DK:                                                                                              \
+        if (a.nsplit > 1)                                                                                 \
+            hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, DK, 1, NW, true>), dim3(grid), dim3(NW * 64), 0, st, a); \
+        else                                                                                              \
+            hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, DK, 1, NW, false>), dim3(grid), dim3(NW * 64), 0, st, a); \
         break;
         FTA_FWD(32, 1, 8)
         case 64:
@@ -2244,7 +2281,7 @@ int launch_fwd_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
             else if (pipe_ok)
                 hipLaunchKernelGGL((fta_sparse_fwd_pipe_kernel<DT, 64, 8, false>), dim3(grid), dim3(512), 0, st, a);
             else
-                hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, 64, 1, 8>), dim3(grid), dim3(512), 0, st, a);
+                hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, 64, 1, 8, false>), dim3(grid), dim3(512), 0, st, a);
             break;
         FTA_FWD(96, 1, 8)
         case 128:
@@ -2253,22 +2290,25 @@ int launch_fwd_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
             else if (pipe_ok)
                 hipLaunchKernelGGL((fta_sparse_fwd_pipe_kernel<DT, 128, 8, false>), dim3(grid), dim3(512), 0, st, a);
             else
-                hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, 128, 1, 8>), dim3(grid), dim3(512), 0, st, a);
+                hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, 128, 1, 8, false>), dim3(grid), dim3(512), 0, st, a);
             break;
-        FTA_FWD(160, 1, 8)
-        FTA_FWD(256, 1, 4)
+        FTA_FWD_WIDE(160, 8)
+        FTA_FWD_WIDE(256, 4)
 #undef FTA_FWD
+#undef FTA_FWD_WIDE
         default:
             return fta::arg_error("sparse_attn: unsupported head dim");
     }
     int rc = fta::check_launch("fta_sparse_fwd_kernel");
-    if (rc != FTA_OK || !(pipe_ok && a.nsplit > 1)) return rc;
+    if (rc != FTA_OK || a.nsplit <= 1) return rc;
     const int64_t threads = (int64_t)a.nbh * a.N * (Dk / 8);
     const unsigned blocks = (unsigned)((threads + 255) / 256);
-    if (Dk == 64)
-        hipLaunchKernelGGL((fta_fwd_combine_kernel<DT, 64>), dim3(blocks), dim3(256), 0, st, a);
-    else
-        hipLaunchKernelGGL((fta_fwd_combine_kernel<DT, 128>), dim3(blocks), dim3(256), 0, st, a);
+    switch (Dk) {
+        case 64: hipLaunchKernelGGL((fta_fwd_combine_kernel<DT, 64>), dim3(blocks), dim3(256), 0, st, a); break;
+        case 128: hipLaunchKernelGGL((fta_fwd_combine_kernel<DT, 128>), dim3(blocks), dim3(256), 0, st, a); break;
+        case 160: hipLaunchKernelGGL((fta_fwd_combine_kernel<DT, 160>), dim3(blocks), dim3(256), 0, st, a); break;
+        default: hipLaunchKernelGGL((fta_fwd_combine_kernel<DT, 256>), dim3(blocks), dim3(256), 0, st, a); break;
+    }
     return fta::check_launch("fta_fwd_combine_kernel");
 }
 
@@ -2420,12 +2460,15 @@ size_t fwd_bytes(int B, int H) { return fta::align_up((size_t)B * H * (2 + 64) *
 
 // Forward parts per workgroup.  A grid of fewer than 128 workgroups (under half
 // the CUs) is bound by each workgroup's sequential union walk, not by the chip:
-// the pipelined kernel then splits every walk into up to 4 parts (256 / grid)
-// and fta_fwd_combine_kernel merges them.
+// every walk is then split into up to 4 parts (256 / grid) and
+// fta_fwd_combine_kernel merges them.  At D = 256 the workgroups are half as long
+// (128 queries) and 128 of them still leave half the CUs idle: N2048 H8 D256, lists of
+// every block, 139 us unsplit, 81 + 9 us in two parts.
 int fwd_nsplit(int B, int H, const Geo& G) {
-    if (!(G.Dk == 64 || G.Dk == 128) || G.Mkv < 8) return 1;
-    const int64_t wgs = (int64_t)((G.Npq + 255) / 256) * B * H;
-    if (wgs >= 128) return 1;
+    if (!(G.Dk == 64 || G.Dk == 128 || G.Dk == 160 || G.Dk == 256) || G.Mkv < 8) return 1;
+    const int rows = (G.Dk == 256) ? 128 : 256;  // queries per workgroup
+    const int64_t wgs = (int64_t)((G.Npq + rows - 1) / rows) * B * H;
+    if (wgs >= ((G.Dk == 256) ? 129 : 128)) return 1;
     const int64_t ns = 256 / wgs;
     return (int)(ns > 4 ? 4 : ns < 2 ? 2 : ns);
 }
@@ -2452,6 +2495,9 @@ size_t dq_split_bytes(int B, int H, const Geo& G, int ns) {
     if (ns <= 1) return 0;
     return fta::align_up((size_t)ns * B * H * G.Npq * G.Dk * sizeof(float));
 }
+
+// dK/dV workgroups of the split kernel that the chip holds at once
+int64_t dkv_slots(const Geo& G) { return 256 * ((G.Dk <= 64) ? 3 : (G.Dk <= 128) ? 2 : 1); }
 
 // dK/dV parts of the split kernel (64-key blocks, D 64 / 128 / 256) on small
 // grids: fewer workgroups than the CUs hold (two per CU, one at D = 256) get
@@ -2554,11 +2600,11 @@ int fta_sparse_attn_fwd_gqa(const void* q, const int64_t* q_strides, const void*
     a.Hk = Hk;
     a.G = H / Hk;
     a.wg_per_bh = (G.Npq + 32 * T - 1) / (32 * T);
-    // split walks (small grids, pipelined kernel, workspace for the parts)
+    // split walks (small grids, workspace for the parts)
     const int ns = fwd_nsplit(B, H, G);
     const bool split = ns > 1 && workspace != nullptr &&
-                       workspace_bytes >= fwd_bytes(B, H) + split_bytes(B, H, G, ns) && narrow_stride(k_strides[2]) &&
-                       narrow_stride(v_strides[2]);
+                       workspace_bytes >= fwd_bytes(B, H) + split_bytes(B, H, G, ns) &&
+                       (G.Dk > 128 || (narrow_stride(k_strides[2]) && narrow_stride(v_strides[2])));
     a.nsplit = split ? ns : 1;
     a.nbh = B * H;
     a.npq = G.Npq;
@@ -2634,11 +2680,11 @@ int bwd_common(AttnArgs& a, Geo& G, const void* q, const int64_t* q_strides, con
 
 // 64-key blocks at D 64 / 128 / 256 (the split dK/dV kernel) run in the launch
 // order of fta_kv_order_kernel and the head placement of fta_head_balance_kernel,
-// except on grids that split (dkv_nsplit: all their workgroups run at once, so the
-// order cannot change the time; the two launches took 10 of 199 us at N2048 H8 D128)
+// except where all workgroups run at once (the order cannot change the time; the two
+// launches took 10 of 199 us at N2048 H8 D128)
 bool uses_kv_order(int B, int Hk, int kv_block_size, const Geo& G) {
     return kv_block_size > 32 && kv_block_size <= 64 && (G.Dk == 64 || G.Dk == 128 || G.Dk == 256) &&
-           G.Mkv <= 4096 && dkv_nsplit(B, Hk, kv_block_size, G) == 1;
+           G.Mkv <= 4096 && (int64_t)G.Mkv * B * Hk > dkv_slots(G);
 }
 
 // the head placement fta_sparse_attn_bwd_dkv left in the workspace (null if it made none)

@@ -88,3 +88,42 @@ def test_list_loads(W, offset):
         res.append([o.detach(), lse, *torch.autograd.grad(o, (ql, kl, vl), do)])
     for x, y in zip(*res):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("case", [
+    # B, N, H, D, g, b, q padding, kv padding, W, dtype
+    (1, 1030, 2, 256, 32, 64, (3, 23), (13, 45), 10, torch.bfloat16),  # 9 blocks a workgroup, 4 parts
+    (1, 1000, 2, 160, 16, 64, (0, 8), (24, 0), 3, torch.float16),  # parts of one block, and empty ones
+    (1, 600, 1, 192, 48, 160, (0, 24), (0, 40), 2, torch.bfloat16),  # 4 blocks: not split
+], ids=lambda c: f"N{c[1]}D{c[3]}b{c[5]}W{c[8]}")
+def test_wide_head_split_forward(case):
+    """Heads of more than 128 columns split the forward's walks on small grids too:
+    against the same call without a workspace (unsplit), lse to 1e-5 and o to one 16-bit
+    rounding step of the largest probability's weight (the parts round P against their
+    own maxima), and against the oracle."""
+    from flash_topk_attn_v2 import _lib
+
+    B, N, H, D, g, b, qpad, kvpad, W, dt = case
+    say(f"[wide split] {case}")
+    QM, M = (qpad[0] + N + qpad[1]) // g, (kvpad[0] + N + kvpad[1]) // b
+    merged = _random_merged(B, H, QM, W, M, 21)
+    tm = torch.from_numpy(merged).cuda()
+    q, k, v = (rand((B, N, H * D), 22 + i, dt, "cuda") for i in range(3))
+    L = _lib.lib()
+    splits = L.fta_sparse_attn_fwd_splits(B, H, N, D, g, b, *qpad, *kvpad)
+    assert (splits > 1) == (M >= 8)
+    o, lse = fta.flash_topk_attn(q, k, v, tm, None, H, g, b, None, None, kvpad, qpad)
+    st = _lib.i64arr((N * H * D, D, H * D))
+    o2, lse2 = torch.empty_like(o), torch.empty_like(lse)
+    _lib.check(L.fta_sparse_attn_fwd_gqa(q.data_ptr(), st, k.data_ptr(), st, v.data_ptr(), st, _lib.dtype_code(dt), B,
+                                         H, H, N, D, tm.data_ptr(), QM, W, g, b, *qpad, *kvpad, D ** -0.5,
+                                         o2.data_ptr(), st, lse2.data_ptr(), None, 0,
+                                         torch.cuda.current_stream().cuda_stream), "fta_sparse_attn_fwd_gqa")
+    torch.cuda.synchronize()
+    assert torch.equal(torch.isinf(lse), torch.isinf(lse2))
+    fin = torch.isfinite(lse2)
+    assert torch.allclose(lse[fin], lse2[fin], rtol=1e-5, atol=1e-5)
+    # |v| <= 6 here, sum of P = 1 after division: rounding P twice differently moves o by
+    # at most 2 * 2^-9 (bf16) * 6, and the two stored outputs by one step each
+    assert (o.float() - o2.float()).abs().max() <= 2 * 2.0**-9 * 6 + 2 * 2.0**-8 * o2.float().abs().max()
+    check_attn_vs_oracle(q, k, v, None, o, lse, merged, H, g, b, qpad, kvpad, dt)
