@@ -443,7 +443,7 @@ __global__ __launch_bounds__(NW * 64, 1) void fta_sparse_fwd_kernel(AttnArgs a) 
 // scheduling fences: left alone the compiler either keeps a whole chunk's fragments
 // in registers (156 at D = 64) or waits out one LDS latency per MFMA.  B2 N8192 H16
 // D64 fp16, lists of every block: 0.80 -> 0.66 ms; one list of 16 blocks per query:
-// 0.74 -> 0.61 ms (whole call); B1 N16384 H16 D128 dense lists: 1.95 -> 1.88 ms.
+// 0.74 -> 0.59-0.62 ms (whole call, with its list preparation); B1 N16384 H16 D128 dense lists: 1.95 -> 1.88 ms.
 // ----------------------------------------------------------------------------
 template <int D, int NW>
 struct FwdPipeShape {
@@ -2267,13 +2267,6 @@ int launch_fwd_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
     case DK:                                                                                              \
         hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, DK, TPW, NW, false>), dim3(grid), dim3(NW * 64), 0, st, a); \
         break;
-#define FTA_FWD_WIDE(DK, NW)                                                                              \
-    case DK:                                                                                              \
-        if (a.nsplit > 1)                                                                                 \
-            hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, DK, 1, NW, true>), dim3(grid), dim3(NW * 64), 0, st, a); \
-        else                                                                                              \
-            hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, DK, 1, NW, false>), dim3(grid), dim3(NW * 64), 0, st, a); \
-        break;
         FTA_FWD(32, 1, 8)
         case 64:
             if (pipe_ok && a.nsplit > 1)
@@ -2292,10 +2285,14 @@ int launch_fwd_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
             else
                 hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, 128, 1, 8, false>), dim3(grid), dim3(512), 0, st, a);
             break;
-        FTA_FWD_WIDE(160, 8)
-        FTA_FWD_WIDE(256, 4)
+        FTA_FWD(160, 1, 8)
+        case 256:
+            if (a.nsplit > 1)
+                hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, 256, 1, 4, true>), dim3(grid), dim3(256), 0, st, a);
+            else
+                hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, 256, 1, 4, false>), dim3(grid), dim3(256), 0, st, a);
+            break;
 #undef FTA_FWD
-#undef FTA_FWD_WIDE
         default:
             return fta::arg_error("sparse_attn: unsupported head dim");
     }
@@ -2306,7 +2303,6 @@ int launch_fwd_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
     switch (Dk) {
         case 64: hipLaunchKernelGGL((fta_fwd_combine_kernel<DT, 64>), dim3(blocks), dim3(256), 0, st, a); break;
         case 128: hipLaunchKernelGGL((fta_fwd_combine_kernel<DT, 128>), dim3(blocks), dim3(256), 0, st, a); break;
-        case 160: hipLaunchKernelGGL((fta_fwd_combine_kernel<DT, 160>), dim3(blocks), dim3(256), 0, st, a); break;
         default: hipLaunchKernelGGL((fta_fwd_combine_kernel<DT, 256>), dim3(blocks), dim3(256), 0, st, a); break;
     }
     return fta::check_launch("fta_fwd_combine_kernel");
@@ -2463,9 +2459,9 @@ size_t fwd_bytes(int B, int H) { return fta::align_up((size_t)B * H * (2 + 64) *
 // every walk is then split into up to 4 parts (256 / grid) and
 // fta_fwd_combine_kernel merges them.  At D = 256 the workgroups are half as long
 // (128 queries) and 128 of them still leave half the CUs idle: N2048 H8 D256, lists of
-// every block, 139 us unsplit, 81 + 9 us in two parts.
+// every block, 139 us unsplit, 81 + 9 us in two parts.  D = 160 is never split.
 int fwd_nsplit(int B, int H, const Geo& G) {
-    if (!(G.Dk == 64 || G.Dk == 128 || G.Dk == 160 || G.Dk == 256) || G.Mkv < 8) return 1;
+    if (!(G.Dk == 64 || G.Dk == 128 || G.Dk == 256) || G.Mkv < 8) return 1;
     const int rows = (G.Dk == 256) ? 128 : 256;  // queries per workgroup
     const int64_t wgs = (int64_t)((G.Npq + rows - 1) / rows) * B * H;
     if (wgs >= ((G.Dk == 256) ? 129 : 128)) return 1;
@@ -2500,7 +2496,7 @@ size_t dq_split_bytes(int B, int H, const Geo& G, int ns) {
 int64_t dkv_slots(const Geo& G) { return 256 * ((G.Dk <= 64) ? 3 : (G.Dk <= 128) ? 2 : 1); }
 
 // dK/dV parts of the split kernel (64-key blocks, D 64 / 128 / 256) on small
-// grids: fewer workgroups than the CUs hold (two per CU, one at D = 256) get
+// grids: fewer than two workgroups per CU (one at D = 256) get
 // up to 4 parts per KV block; [dK, dV][part][b * Hk][KV block * 64 + key][Dk]
 // fp32, after bwd_bytes (dQ's parts reuse the same bytes after dK/dV is done)
 int dkv_nsplit(int B, int Hk, int kv_block_size, const Geo& G) {

@@ -100,7 +100,7 @@ int fta_topk_select(const float* block_scores, int64_t rows, int M, int64_t stri
  * returns the recommended size for one call's geometry (0 for an invalid one),
  * assuming a K token stride of at most 2^24 elements.
  *
- * b = 64 or 128, D <= 128 and at most 32 blocks per query run
+ * b = 48, 64 or 128, D <= 128 and at most 32 blocks per query run
  * on candidate streams: chunks of 1024 entries taken from a pool in the
  * workspace, one chunk per 64 queries plus a shared remainder, sized for the
  * expected number of entries (m_out (1 + 2 ln(M / m_out)) per query; 1.17e9
@@ -109,7 +109,8 @@ int fta_topk_select(const float* block_scores, int64_t rows, int M, int64_t stri
  * fta_topk_score_workspace_min bytes (one chunk per 64 queries plus the fixed
  * parts) is accepted: the 256-query tiles whose streams do not fit are scored
  * and selected again by a fallback kernel (same results, more time).  Other
- * geometries store the [B][H][M][N] per-block values.
+ * geometries store the [B][H][M][N] per-block values; so does b = 48 in a workspace
+ * below that least size that holds them.
  */
 size_t fta_topk_score_workspace_size(int B, int H, int N, int M);
 size_t fta_topk_score_workspace_size_ex(int B, int H, int N, int D, int score_block_size, int pad_head,
@@ -244,7 +245,7 @@ size_t fta_sparse_attn_fwd_workspace_size(int B, int H, int N, int D, int q_bloc
 /*
  * Parts per workgroup walk of the forward with its workspace for this
  * geometry (0 for an invalid one): 1, or 2-4 when the grid has fewer than 128
- * workgroups and D <= 128.  Then each workgroup's walk over the union of its
+ * workgroups and D <= 128, or at most 128 and D > 160.  Then each workgroup's walk over the union of its
  * q-blocks' lists (ascending, per 512-block segment) is split into that many
  * contiguous ranges, each with its own online-softmax anchor, and a combine
  * kernel merges the parts' (O, max, sum).  No counterpart in the reference
@@ -303,8 +304,8 @@ int fta_sparse_attn_fwd_gqa(const void* q, const int64_t* q_strides, const void*
 /*
  * Backward workspace: the membership bitmap, the lse in log2 units and the
  * dK/dV launch order, plus, on small grids, room for split walks (one region,
- * used by dK/dV and then by dQ): dK/dV with fewer workgroups than the GPU holds
- * at once (64-key blocks at D 64 / 128 / 256) and dQ with fewer than 128
+ * used by dK/dV and then by dQ): dK/dV with fewer than 512 workgroups (256 at
+ * D 256; 64-key blocks at D 64 / 128 / 256) and dQ with fewer than 128
  * workgroups (at most 128 at D 160 / 256) walk their lists in 2-4 parts whose
  * fp32 sums are added by a combine kernel.  A smaller workspace (at least the bitmap, lse and order)
  * runs the walks unsplit: the results then differ only in fp32 summation

@@ -93,11 +93,12 @@ def test_list_loads(W, offset):
 @pytest.mark.parametrize("case", [
     # B, N, H, D, g, b, q padding, kv padding, W, dtype
     (1, 1030, 2, 256, 32, 64, (3, 23), (13, 45), 10, torch.bfloat16),  # 9 blocks a workgroup, 4 parts
-    (1, 1000, 2, 160, 16, 64, (0, 8), (24, 0), 3, torch.float16),  # parts of one block, and empty ones
+    (1, 1000, 2, 224, 16, 64, (0, 8), (24, 0), 3, torch.float16),  # 224 columns run as 256; short lists
+    (1, 1000, 2, 160, 16, 64, (0, 8), (24, 0), 3, torch.float16),  # not split at D = 160
     (1, 600, 1, 192, 48, 160, (0, 24), (0, 40), 2, torch.bfloat16),  # 4 blocks: not split
 ], ids=lambda c: f"N{c[1]}D{c[3]}b{c[5]}W{c[8]}")
 def test_wide_head_split_forward(case):
-    """Heads of more than 128 columns split the forward's walks on small grids too:
+    """Heads of more than 160 columns split the forward's walks on small grids too:
     against the same call without a workspace (unsplit), lse to 1e-5 and o to one 16-bit
     rounding step of the largest probability's weight (the parts round P against their
     own maxima), and against the oracle."""
@@ -111,7 +112,7 @@ def test_wide_head_split_forward(case):
     q, k, v = (rand((B, N, H * D), 22 + i, dt, "cuda") for i in range(3))
     L = _lib.lib()
     splits = L.fta_sparse_attn_fwd_splits(B, H, N, D, g, b, *qpad, *kvpad)
-    assert (splits > 1) == (M >= 8)
+    assert (splits > 1) == (M >= 8 and D > 160)
     o, lse = fta.flash_topk_attn(q, k, v, tm, None, H, g, b, None, None, kvpad, qpad)
     st = _lib.i64arr((N * H * D, D, H * D))
     o2, lse2 = torch.empty_like(o), torch.empty_like(lse)
