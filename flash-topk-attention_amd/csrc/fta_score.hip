@@ -595,13 +595,12 @@ __device__ __forceinline__ uint32_t fta_f2h2(float lo, float hi) {
 // formed at its last chunk from the chunk totals, all taken against the row's
 // running reference R (an exact-path re-reference inside a block rescales the
 // block's earlier chunks, as it rescales the row total).
-// BK = 48 (b = 48, SB = 1): a chunk is one block of 48 keys.  Its second half's
+// BK = 48 (b = 48, SB = 1, NG = 0): a chunk is one block of 48 keys.  Its second half's
 // scores are 16 keys, registers 0 .. 7 of each lane in the 32 x 32 layout, so only
 // those eight exponentials are formed; the products of the 16 rows past them are
 // wasted (a quarter of the MFMAs) and their results dropped.  The values are those of
 // the unpipelined kernel bit for bit (its masked terms add exact zeros).  B1 N4032 H32
-// D128 top-16: scoring kernel 0.328 -> 0.183 ms, with streams in place of per-block
-// values (selector 0.078 -> 0.059 ms).
+// D128: scoring kernel 0.328 -> 0.183 ms; whole top-16 call 365 -> 238 us.
 template <int DT, int D, int NG, int GT = 2, bool GH = false, int SB = 1, int BK = 64>
 __device__ __forceinline__ void fta_score_tile(const ScoreArgs& a, const int wg) {
     const uint16_t* __restrict__ q = a.q;
@@ -620,7 +619,8 @@ __device__ __forceinline__ void fta_score_tile(const ScoreArgs& a, const int wg)
     __shared__ __align__(1024) unsigned char sK[NBUF][Sh::BUF_B];
     static_assert(GT == 2 || GT == 4, "group top-2 or top-4");
     static_assert(!GH || GT == 4, "fp16 group state holds four keys");
-    static_assert(SB == 1 || (SB == 2 && BK == 64), "blocks of 48, 64 or 128 keys");
+    static_assert((SB == 1 && BK == 64) || (SB == 2 && BK == 64) || (SB == 1 && BK == 48 && !STREAM),
+                  "blocks of 64 or 128 keys, or of 48 without streams");
     static_assert(BK == 64 || BK == 48, "16-key granules of a chunk's second half");
     constexpr int NE1 = (BK - 32) / 2;  // scores per lane and query tile of a chunk's second half
     constexpr int GB = GT * (GH ? 2 : 4);  // bytes per (group, query)
@@ -1782,7 +1782,7 @@ __global__ void fta_stream_reset_kernel(int* __restrict__ ctrs) {
 // top-k from the slot with the selector of the per-block-value path.  The
 // results equal the stream path's (both selectors are exact); only the time
 // differs.
-template <int DT, int D, int KB, int SB, int BK>
+template <int DT, int D, int KB, int SB>
 __global__ __launch_bounds__(256, 1) void fta_stream_fallback_kernel(ScoreArgs a, const int* __restrict__ ovf_list,
                                                                     const int* __restrict__ ovf_cnt,
                                                                     float* __restrict__ slots, int m_out,
@@ -1800,7 +1800,7 @@ __global__ __launch_bounds__(256, 1) void fta_stream_fallback_kernel(ScoreArgs a
     for (int r = blockIdx.x; r < n; r += gridDim.x) {
         const int tile = __builtin_amdgcn_readfirstlane(ovf_list[r]);
         if ((unsigned)tile >= (unsigned)a.total) continue;  // workgroup-uniform
-        fta_score_tile<DT, D, 0, 2, false, SB, BK>(a, tile);
+        fta_score_tile<DT, D, 0, 2, false, SB>(a, tile);
         __syncthreads();  // the slot is complete
         const int bh = tile / a.qtiles, qt = tile - bh * a.qtiles;
         const int64_t r0 = (int64_t)bh * a.N + qt * 256;
@@ -1908,6 +1908,13 @@ bool score_pipe_ok(int bsz, int Dk, const int64_t* ks) {
     return (bsz == 48 || bsz == 64 || bsz == 128) && Dk <= 128 && ks[2] >= 0 && ks[2] <= (1 << 24);
 }
 
+// Candidate streams serve b = 64 and 128.  48-key blocks keep their per-block values:
+// the streams gain 4-5% at most (N4032 H32 D128 top-16 229 us against 238, N15984 H4
+// D64 top-32 459 against 481), and where their pool overflows the fallback kernel
+// scores the tiles again (iid data, N916 H32 D96 top-8, 116 us against 44; block
+// scores that rise along the sequence, N4032 H16 D128, 853 against 176).
+bool score_streams_ok(int bsz, int Dk, const int64_t* ks) { return bsz != 48 && score_pipe_ok(bsz, Dk, ks); }
+
 // Candidate streams of the pipelined kernel (STREAM = true), laid out in the
 // workspace by stream_layout: per-wave entry counts, chunk tables, the two
 // counters (pool chunks taken, fallback tiles), the fallback tile list, row
@@ -1977,7 +1984,8 @@ int launch_score_lse_dt(const void* q, const void* k, int B, int H, int N, int D
     const int total = qtiles * B * H;
     const float c = scale * 1.4426950408889634f;
     const bool pipe = score_pipe_ok(bsz, Dk, ks);
-    if (sb.pool != nullptr && !pipe) return fta::arg_error("block_score: candidate streams need the pipelined kernel");
+    if (sb.pool != nullptr && !score_streams_ok(bsz, Dk, ks))
+        return fta::arg_error("block_score: candidate streams need the pipelined kernel");
     if (sb.pool != nullptr) {
         hipLaunchKernelGGL(fta_stream_reset_kernel, dim3(1), dim3(64), 0, st, sb.ctrs);
         int rc = fta::check_launch("fta_stream_reset_kernel");
@@ -1992,8 +2000,6 @@ int launch_score_lse_dt(const void* q, const void* k, int B, int H, int N, int D
     do {                                                                                                   \
         if (bsz == 64)                                                                                     \
             FTA_LAUNCH_PIPE_SB(DK, NG, GT, GH, 1, 64);                                                     \
-        else if (bsz == 48)                                                                                \
-            FTA_LAUNCH_PIPE_SB(DK, NG, GT, GH, 1, 48);                                                     \
         else                                                                                               \
             FTA_LAUNCH_PIPE_SB(DK, NG, GT, GH, 2, 64);                                                     \
     } while (0)
@@ -2004,6 +2010,8 @@ int launch_score_lse_dt(const void* q, const void* k, int B, int H, int N, int D
         FTA_LAUNCH_PIPE(DK, 4, 4, false);                                                                  \
     else if (pipe && sb.pool != nullptr)                                                                   \
         FTA_LAUNCH_PIPE(DK, 8, 4, true);                                                                   \
+    else if (pipe && bsz == 48)                                                                            \
+        FTA_LAUNCH_PIPE_SB(DK, 0, 2, false, 1, 48);                                                        \
     else if (pipe)                                                                                         \
         FTA_LAUNCH_PIPE(DK, 0, 2, false);                                                                  \
     else if (bsz <= 64)                                                                                    \
@@ -2201,7 +2209,7 @@ size_t fta_topk_score_workspace_size_ex(int B, int H, int N, int D, int score_bl
         return 0;
     const int m_out = (max_topk > 0 && max_topk < M) ? max_topk : M;
     const int64_t ks[3] = {0, 0, 0};  // a token stride within the pipelined kernel's range
-    if (m_out <= kStreamMaxTopk && score_pipe_ok(score_block_size, fta::kernel_head_dim(D), ks))
+    if (m_out <= kStreamMaxTopk && score_streams_ok(score_block_size, fta::kernel_head_dim(D), ks))
         return stream_rec_bytes(B, H, N, M, m_out);
     return full_bytes(B, H, N, M);
 }
@@ -2213,7 +2221,7 @@ size_t fta_topk_score_workspace_min(int B, int H, int N, int D, int score_block_
         return 0;
     const int m_out = (max_topk > 0 && max_topk < M) ? max_topk : M;
     const int64_t ks[3] = {0, 0, 0};
-    if (m_out <= kStreamMaxTopk && score_pipe_ok(score_block_size, fta::kernel_head_dim(D), ks))
+    if (m_out <= kStreamMaxTopk && score_streams_ok(score_block_size, fta::kernel_head_dim(D), ks))
         return stream_min_bytes(B, H, N, M);
     return full_bytes(B, H, N, M);
 }
@@ -2274,21 +2282,17 @@ int launch_stream_select_dt(const ScoreArgs& sa, int Dk, const StreamBufs& sb, i
     int rc = fta::check_launch("fta_topk_stream_kernel");
     if (rc != FTA_OK) return rc;
     const int grid = sa.total < kStreamSlots ? sa.total : kStreamSlots;
-#define FTA_LAUNCH_FALLBACK(DK, SB, BK)                                                                         \
-    hipLaunchKernelGGL((fta_stream_fallback_kernel<DT, DK, 32, SB, BK>), dim3(grid), dim3(256), 0, s, sa,         \
-                       sb.ovf_list, sb.ctrs + 1, sb.slots, m_out, threshold, idx, raw, avg)
+#define FTA_LAUNCH_FALLBACK(DK, SB)                                                                             \
+    hipLaunchKernelGGL((fta_stream_fallback_kernel<DT, DK, 32, SB>), dim3(grid), dim3(256), 0, s, sa, sb.ovf_list, \
+                       sb.ctrs + 1, sb.slots, m_out, threshold, idx, raw, avg)
     if (Dk <= 64 && sa.bsz == 64)
-        FTA_LAUNCH_FALLBACK(64, 1, 64);
-    else if (Dk <= 64 && sa.bsz == 48)
-        FTA_LAUNCH_FALLBACK(64, 1, 48);
+        FTA_LAUNCH_FALLBACK(64, 1);
     else if (Dk <= 64)
-        FTA_LAUNCH_FALLBACK(64, 2, 64);
+        FTA_LAUNCH_FALLBACK(64, 2);
     else if (sa.bsz == 64)
-        FTA_LAUNCH_FALLBACK(128, 1, 64);
-    else if (sa.bsz == 48)
-        FTA_LAUNCH_FALLBACK(128, 1, 48);
+        FTA_LAUNCH_FALLBACK(128, 1);
     else
-        FTA_LAUNCH_FALLBACK(128, 2, 64);
+        FTA_LAUNCH_FALLBACK(128, 2);
 #undef FTA_LAUNCH_FALLBACK
     return fta::check_launch("fta_stream_fallback_kernel");
 }
@@ -2302,10 +2306,7 @@ int topk_score_checks(int B, int H, int N, int D, int bsz, int pad_head, int pad
     if (*M > 4096) return fta::unsupported("topk_score: M exceeds 4096");
     if (max_topk < 0) return fta::arg_error("topk_score: max_topk must be >= 0");
     *m_out = (max_topk > 0 && max_topk < *M) ? max_topk : *M;
-    *streams = *m_out <= kStreamMaxTopk && score_pipe_ok(bsz, fta::kernel_head_dim(D), k_strides);
-    // b = 48 also takes the per-block-value path, in a workspace that holds only that
-    // (callers that sized it so before these blocks had streams)
-    if (bsz == 48 && *streams && workspace_bytes < stream_min_bytes(B, H, N, *M)) *streams = false;
+    *streams = *m_out <= kStreamMaxTopk && score_streams_ok(bsz, fta::kernel_head_dim(D), k_strides);
     const size_t need = *streams ? stream_min_bytes(B, H, N, *M) : full_bytes(B, H, N, *M);
     if (workspace_bytes < need)
         return fta::arg_error("topk_score: workspace too small (see fta_topk_score_workspace_size_ex)");
@@ -2341,7 +2342,7 @@ int fta_topk_score_candidates(const void* q, const void* k, int dtype, int B, in
     int st = topk_score_checks(B, H, N, D, score_block_size, pad_head, pad_tail, max_topk, k_strides,
                                workspace_bytes, &M, &m_out, &streams);
     if (st != FTA_OK) return st;
-    if (!streams || score_block_size == 48)
+    if (!streams)
         return fta::unsupported("topk_score_candidates: needs b = 64 or 128, D <= 128 and at most 32 blocks per query");
     float* row_lse = nullptr;
     const StreamBufs sb = stream_layout(workspace, workspace_bytes, B, H, N, M, m_out, &row_lse);
@@ -2361,7 +2362,7 @@ int fta_topk_select_candidates(const void* q, const void* k, int dtype, int B, i
     int st = topk_score_checks(B, H, N, D, score_block_size, pad_head, pad_tail, max_topk, k_strides,
                                workspace_bytes, &M, &m_out, &streams);
     if (st != FTA_OK) return st;
-    if (!streams || score_block_size == 48)
+    if (!streams)
         return fta::unsupported("topk_select_candidates: needs b = 64 or 128, D <= 128 and at most 32 blocks per query");
     if (!topk_indices || !topk_raw || !topk_avg) return fta::arg_error("topk_select_candidates: null pointer");
     return stream_select(q, k, dtype, B, H, N, D, q_strides, k_strides, score_block_size, pad_head, pad_tail, scale,

@@ -100,7 +100,7 @@ int fta_topk_select(const float* block_scores, int64_t rows, int M, int64_t stri
  * returns the recommended size for one call's geometry (0 for an invalid one),
  * assuming a K token stride of at most 2^24 elements.
  *
- * b = 48, 64 or 128, D <= 128 and at most 32 blocks per query run
+ * b = 64 or 128, D <= 128 and at most 32 blocks per query run
  * on candidate streams: chunks of 1024 entries taken from a pool in the
  * workspace, one chunk per 64 queries plus a shared remainder, sized for the
  * expected number of entries (m_out (1 + 2 ln(M / m_out)) per query; 1.17e9
@@ -109,8 +109,7 @@ int fta_topk_select(const float* block_scores, int64_t rows, int M, int64_t stri
  * fta_topk_score_workspace_min bytes (one chunk per 64 queries plus the fixed
  * parts) is accepted: the 256-query tiles whose streams do not fit are scored
  * and selected again by a fallback kernel (same results, more time).  Other
- * geometries store the [B][H][M][N] per-block values; so does b = 48 in a workspace
- * below that least size that holds them.
+ * geometries store the [B][H][M][N] per-block values.
  */
 size_t fta_topk_score_workspace_size(int B, int H, int N, int M);
 size_t fta_topk_score_workspace_size_ex(int B, int H, int N, int D, int score_block_size, int pad_head,

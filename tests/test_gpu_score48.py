@@ -1,4 +1,4 @@
-"""Score blocks of 48 keys on the pipelined scorer and its candidate streams."""
+"""Score blocks of 48 keys on the pipelined scorer, with per-block values."""
 
 import numpy as np
 import pytest
@@ -18,7 +18,7 @@ CASES = [
     (4032, 2, 64, (0, 0), 8, 0.9, "decreasing"),
     (4032, 1, 128, (0, 0), 32, 1.0, "ties"),
     (4032, 2, 128, (0, 0), 16, 1.0, "jump"),  # the exact path inside the unrolled loop
-    (4032, 1, 64, (0, 0), 24, 2.0, "cliff"),  # averages that underflow: the fallback kernel
+    (4032, 1, 64, (0, 0), 24, 2.0, "cliff"),  # averages that underflow
     (4032, 2, 128, (0, 0), 16, 2.0, "step"),
     (4032, 2, 64, (0, 0), 32, 0.95, "uniform"),
     (5167, 2, 64, (40, 25), 5, 0.9, "peaked"),  # edge blocks of 8 and 23 keys
@@ -39,7 +39,7 @@ def _check(out, scores, thr, topk, pad):
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: f"N{c[0]}D{c[2]}k{c[4]}{c[6]}p{c[3][0]}")
-def test_streams_b48(case):
+def test_scores_b48(case):
     """Block scores against the float64 oracle (rtol 2e-4, as for every block size), and
     the fused top-k equal to the selection over them bit for bit."""
     N, H, D, pad, topk, thr, pattern = case
@@ -53,29 +53,33 @@ def test_streams_b48(case):
 
 
 @pytest.mark.parametrize("pattern,D", [("increasing", 128), ("ties", 64)])
-def test_workspaces_b48(pattern, D):
-    """With the least workspace the tiles overflow into the fallback kernel; with one that
-    holds only per-block values those are used: the same lists.  The two halves of the
-    stream path keep refusing 48-key blocks."""
+def test_workspace_b48(pattern, D):
+    """The sizes are those of the per-block values, and a workspace of that size serves
+    any K token stride: the pipelined scorer (tokens in order) and the general one (tokens
+    stored last to first) give the same lists.  The two halves of the stream path refuse
+    48-key blocks."""
     from flash_topk_attn_v2 import _lib
 
-    N, H, topk = 4032, 2, 16
+    N, H, topk = 4032, 16, 2
     M = N // 48
-    say(f"[b48 workspaces] {pattern} D{D}")
+    say(f"[b48 workspace] {pattern} D{D}")
     q, k = _pattern_qk(N, H, D, pattern, 43, 48)
-    scores = fta.flash_block_score(q, k, H, 48).cpu().numpy()
     L = _lib.lib()
-    st = _lib.i64arr([N * H * D, D, H * D])
-    stream = torch.cuda.current_stream().cuda_stream
     al = lambda x: (x + 255) // 256 * 256  # noqa: E731
-    values = al(H * M * N * 4) + 2 * al(H * N * 4)
-    least = L.fta_topk_score_workspace_min(1, H, N, D, 48, 0, 0, topk)
-    assert 0 < least < L.fta_topk_score_workspace_size_ex(1, H, N, D, 48, 0, 0, topk)
-    for nbytes in (least, values):
-        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    nbytes = L.fta_topk_score_workspace_size_ex(1, H, N, D, 48, 0, 0, topk)
+    assert nbytes == L.fta_topk_score_workspace_min(1, H, N, D, 48, 0, 0, topk)
+    assert nbytes == al(H * M * N * 4) + 2 * al(H * N * 4)
+    st = _lib.i64arr([N * H * D, D, H * D])
+    back = _lib.i64arr([N * H * D, D, -H * D])
+    kr = k.flip(1).contiguous()
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    want = fta.flash_topk_score(q, k, H, 48, topk)
+    for kp, ks in ((k.data_ptr(), st), (kr.data_ptr() + 2 * (N - 1) * H * D, back)):
         out = [torch.full((1, H, N, topk), 7, dtype=t, device="cuda") for t in (torch.int32, torch.float32, torch.float32)]
-        args = (q.data_ptr(), k.data_ptr(), 0, 1, H, N, D, st, st, 48, 0, 0, D ** -0.5, topk)
+        args = (q.data_ptr(), kp, 0, 1, H, N, D, st, ks, 48, 0, 0, D ** -0.5, topk)
         _lib.check(L.fta_topk_score(*args, 1.0, *(o.data_ptr() for o in out), ws.data_ptr(), nbytes, stream), "score")
         torch.cuda.synchronize()
-        _check(out, scores, 1.0, topk, (0, 0))
-    assert L.fta_topk_score_candidates(*args, ws.data_ptr(), nbytes, stream) == _lib.FTA_ERR_UNSUPPORTED
+        for x, y in zip(out, want):
+            assert torch.equal(x, y)
+        assert L.fta_topk_score_candidates(*args, ws.data_ptr(), nbytes, stream) == _lib.FTA_ERR_UNSUPPORTED
