@@ -615,25 +615,37 @@ __device__ __forceinline__ void fta_each_id(const int32_t* __restrict__ p, int r
 // when q-block qm's merged list holds KV block m.  One workgroup per (bh, qw)
 // builds that word column for every m in LDS (atomicOr there), a chunk of
 // kSelChunk blocks at a time, and writes every word: no global atomics and no
-// separate clearing pass.  The workgroups also form lse2 = lse * log2(e) (n_lse
-// values; the fp32 product that the dK/dV kernel would form per element) if lse is
-// set: it needs no launch of its own.  Latency-bound on small grids (8 workgroups at
-// N2048 H8 g64): 22 -> 8 us there with the loads of fta_each_id, 24 -> 16 us at
-// N32768 H32 g32.
+// separate clearing pass.  Workgroups past the `nsel` of the bitmap form lse2 = lse *
+// log2(e) (n_lse values, kLseChunk each; the fp32 product that the dK/dV kernel would
+// form per element): it needs no launch of its own, and its loads are spread by the
+// number of values, whatever the size of a q-block (formed by the bitmap's workgroups,
+// g / 8 values in turn per thread, a backward at N32768 H8 g1024 took 504 us; 470 so).
+// Latency-bound on small grids (8
+// workgroups at N2048 H8 g64): 22 -> 8 us there with the loads of fta_each_id, 24 ->
+// 16 us at N32768 H32 g32.
 constexpr int kSelChunk = 8192;
+constexpr int kLseChunk = 2048;  // 8 loads in flight per thread
 
 __global__ __launch_bounds__(256) void fta_sel_bitmap_kernel(const int32_t* __restrict__ merged, int QM, int W,
-                                                             int M, int QW, uint32_t* __restrict__ sel,
+                                                             int M, int QW, uint32_t* __restrict__ sel, int nsel,
                                                              const float* __restrict__ lse, float* __restrict__ lse2,
                                                              int64_t n_lse) {
     __shared__ uint32_t bits[kSelChunk];
+    if ((int)blockIdx.x >= nsel) {
+        constexpr int U = kLseChunk / 256;
+        const int64_t i0 = (int64_t)((int)blockIdx.x - nsel) * kLseChunk + threadIdx.x;
+        float v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = (i0 + u * 256 < n_lse) ? lse[i0 + u * 256] : 0.f;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (i0 + u * 256 < n_lse) lse2[i0 + u * 256] = v[u] * 1.4426950408889634f;
+        return;
+    }
     const int64_t bh = blockIdx.x / QW;
     const int qw = (int)(blockIdx.x - bh * QW);
     const int q0 = qw * 32, nq = min(32, QM - q0);
     const int32_t* mp = merged + (bh * QM + q0) * (int64_t)W;
-    if (lse != nullptr)
-        for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_lse; i += (int64_t)gridDim.x * 256)
-            lse2[i] = lse[i] * 1.4426950408889634f;
     for (int m0 = 0; m0 < M; m0 += kSelChunk) {
         const int mn = min(kSelChunk, M - m0);
         for (int i = threadIdx.x; i < mn; i += 256) bits[i] = 0u;
@@ -647,7 +659,6 @@ __global__ __launch_bounds__(256) void fta_sel_bitmap_kernel(const int32_t* __re
         __syncthreads();
     }
 }
-
 
 // One wave per (bh, m): ascending q-block list, -1 fill, count.
 __global__ __launch_bounds__(64) void fta_reverse_lists_kernel(const uint32_t* __restrict__ sel, int QM, int QW,
@@ -778,6 +789,14 @@ __global__ __launch_bounds__(256) void fta_kv_order_kernel(const uint32_t* __res
     }
 }
 
+// The 64-bit value of the lane that DPP control CTRL names (within a row of 16).
+template <int CTRL>
+__device__ __forceinline__ long long fta_dpp64(long long x) {
+    const int lo = __builtin_amdgcn_mov_dpp((int)x, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(x >> 32), CTRL, 0xf, 0xf, true);
+    return ((long long)hi << 32) | (uint32_t)lo;
+}
+
 // XCD placement of the dK/dV heads.  The WGs of head position p run on XCD
 // p / (n / 8) (fta_xcd_remap gives each XCD a contiguous range of the grid), so
 // heads of unequal total work (head_work: selection counts plus setup) leave
@@ -787,14 +806,6 @@ __global__ __launch_bounds__(256) void fta_kv_order_kernel(const uint32_t* __res
 // n not a multiple of 8, or above 4096 heads: identity.
 // With `part` set, each head's work is first formed from its partial counts:
 // head_work[i] = base + scale * sum_j part[i][j] (j < nparts).
-// The 64-bit value of the lane that DPP control CTRL names (within a row of 16).
-template <int CTRL>
-__device__ __forceinline__ long long fta_dpp64(long long x) {
-    const int lo = __builtin_amdgcn_mov_dpp((int)x, CTRL, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(x >> 32), CTRL, 0xf, 0xf, true);
-    return ((long long)hi << 32) | (uint32_t)lo;
-}
-
 __global__ __launch_bounds__(256) void fta_head_balance_kernel(int32_t* __restrict__ head_work,
                                                                const int32_t* __restrict__ part, int nparts,
                                                                int base, int scale, int n,
@@ -1040,9 +1051,11 @@ namespace fta {
 int launch_sel_bitmap(const int32_t* merged, int BH, int QM, int W, int M, uint32_t* sel, const float* lse,
                       float* lse2, int64_t n_lse, hipStream_t st) {
     const int QW = (QM + 31) / 32;
-    if ((int64_t)BH * QW == 0 || M <= 0) return FTA_OK;
-    hipLaunchKernelGGL(fta_sel_bitmap_kernel, dim3((unsigned)((int64_t)BH * QW)), dim3(256), 0, st, merged, QM, W,
-                       M, QW, sel, lse, lse2, n_lse);
+    const int64_t nsel = (int64_t)BH * QW;
+    if (nsel == 0 || M <= 0) return FTA_OK;
+    const int64_t nlse = lse != nullptr ? (n_lse + kLseChunk - 1) / kLseChunk : 0;
+    hipLaunchKernelGGL(fta_sel_bitmap_kernel, dim3((unsigned)(nsel + nlse)), dim3(256), 0, st, merged, QM, W, M, QW,
+                       sel, (int)nsel, lse, lse2, n_lse);
     return check_launch("fta_sel_bitmap_kernel");
 }
 

@@ -128,3 +128,24 @@ def test_wide_head_split_forward(case):
     # at most 2 * 2^-9 (bf16) * 6, and the two stored outputs by one step each
     assert (o.float() - o2.float()).abs().max() <= 2 * 2.0**-9 * 6 + 2 * 2.0**-8 * o2.float().abs().max()
     check_attn_vs_oracle(q, k, v, None, o, lse, merged, H, g, b, qpad, kvpad, dt)
+
+
+@pytest.mark.parametrize("N,H,D,g", [(2500, 3, 64, 256), (1025, 1, 128, 1024), (700, 2, 64, 192)])
+def test_wide_query_blocks(N, H, D, g):
+    """The backward takes q-blocks of any size: blocks of ``g`` queries give the bits of
+    the same lists repeated for blocks of 64 (few bitmap workgroups, log2 lse values in
+    several chunks and in one partly filled one)."""
+    from flash_topk_attn_v2.sparse_attn_bwd import sparse_attn_bwd
+
+    b, W = 64, 4
+    say(f"[wide q-blocks] N{N} H{H} D{D} g{g}")
+    qpad, kvpad = -N % g, -N % b
+    QM, M, q64 = (N + qpad) // g, (N + kvpad) // b, -N % 64
+    lists = torch.from_numpy(_random_merged(1, H, QM, W, M, 7)).cuda()
+    fine = lists.repeat_interleave(g // 64, dim=2)[:, :, :(N + q64) // 64].contiguous()
+    q, k, v, do = (rand((1, N, H * D), 60 + i, torch.bfloat16, "cuda") for i in range(4))
+    o, lse = fta.flash_topk_attn(q, k, v, fine, None, H, 64, b, None, None, (0, kvpad), (0, q64))
+    res = [sparse_attn_bwd(q, k, v, o, do, lse, tm, H, gg, b, D ** -0.5, (0, qp), (0, kvpad))
+           for tm, gg, qp in ((fine, 64, q64), (lists, g, qpad))]
+    for x, y in zip(*res):
+        assert torch.equal(x, y)
