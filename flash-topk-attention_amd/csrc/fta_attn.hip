@@ -1786,10 +1786,13 @@ __global__ __launch_bounds__(TT * CS * 64, 1) void fta_sparse_dkv_kernel(AttnArg
 //
 // Steps: one chunk per step and one barrier.  Role 1 works one chunk behind role 0,
 // so of the chunk in flight only Q is needed early: four Q and three dO tiles hold
-// the live chunks and two steps of gathers, in the LDS that three whole stages and
-// longer mask segments took for one step of gathers.  The list entry and mask of the
-// next step are read one step ahead, P crosses as 16-byte LDS accesses, and the rows
-// a partly selected chunk leaves out are masked with one sign-extended bit each.
+// the live chunks and two steps of gathers, in the LDS that three whole stages took
+// for one step of gathers.  The two tiles are of one KV block, so one mask row serves
+// both and a segment holds 1024 chunks; with half as many a sequence of more than 16384
+// queries restarts every walk (dK/dV of B1 N32768 H32 D128, one block per list of 64
+// queries: 654 us against 551).  The list entry and mask of the next step are read one
+// step ahead, P crosses as 16-byte LDS accesses, and the rows a partly selected chunk
+// leaves out are masked with one sign-extended bit each.
 // What bounds it: each chunk's 16 KB (D = 128) serves only 64 keys, so the gathers
 // (7.4 TB/s from L2 on dense lists) and the matrix pipe (40% busy) share the time.
 // dK/dV on B1 N16384 H16 D128 dense lists 4.41 -> 4.12 ms, B1 N32768 H32 D128 short
@@ -1806,9 +1809,9 @@ struct DkvSplitShape {
     static constexpr int TILE_B = TILE * 16;
     static constexpr int NQ = 4, ND = 3;                // Q and dO tiles in LDS
     static constexpr int WPC = (D <= 64) ? 3 : (D <= 128) ? 2 : 1;  // WGs per CU
-    static constexpr int SEG = 512;                     // chunks per mask segment
+    static constexpr int SEG = kSegC;                   // chunks per mask segment
     static_assert(TILE % NTHR == 0, "whole DMA instructions per wave");
-    static_assert((NQ + ND) * TILE_B + NQ * 256 + 2 * 2 * 32 * 32 * 4 + 2 * SEG * 4 + SEG * 2 + 2 * kBitsW * 4 + 64 <=
+    static_assert((NQ + ND) * TILE_B + NQ * 256 + 2 * 2 * 32 * 32 * 4 + SEG * 4 + SEG * 2 + kBitsW * 4 + 64 <=
                       160 * 1024 / WPC,
                   "WPC WGs per CU");
 };
@@ -1826,9 +1829,9 @@ __global__ __launch_bounds__(256, DkvSplitShape<D>::WPC) void fta_sparse_dkv_spl
     __shared__ __align__(1024) unsigned char sD[Sh::ND][TILE_B];
     __shared__ __align__(1024) float sL[Sh::NQ][64];  // [lse of chunk k, delta of chunk k - 1] at k % 4
     __shared__ float4 sX[2][TT][4][64];  // [step parity][tile][i / 4][lane]: P of the last two steps
-    __shared__ uint32_t sMask[TT][SEG];
+    __shared__ uint32_t sMask[1][SEG];  // both tiles are of one KV block: one membership, one list
     __shared__ uint16_t sList[SEG];
-    __shared__ uint32_t sBits[TT][kBitsW];
+    __shared__ uint32_t sBits[1][kBitsW];
     __shared__ int s_tmp[8];
 
     const int wgi = fta_xcd_remap(blockIdx.x, a.total);
@@ -1851,7 +1854,6 @@ __global__ __launch_bounds__(256, DkvSplitShape<D>::WPC) void fta_sparse_dkv_spl
     const int hf = lane >> 5;
     const int tt = wave & 1;
     const bool hv = (wave >> 1) != 0;  // wave-uniform role: false = K / P / dV, true = V / dS / dK
-    constexpr int Tb = 2;
 
     const int krel = 32 * tt + (lane & 31);  // key of this lane's column, relative to block start
     const int tk = wk * a.kvb - a.kv_pad + krel;
@@ -1875,7 +1877,7 @@ __global__ __launch_bounds__(256, DkvSplitShape<D>::WPC) void fta_sparse_dkv_spl
         }
     }
     // the first query head's membership rows (the staging waits for the K/V loads too)
-    bool bits_lds = fta_stage_kv_bits<TT>(a, b * a.H + hk * a.G, wk, Tb, sBits);
+    bool bits_lds = fta_stage_kv_bits<1>(a, b * a.H + hk * a.G, wk, 1, sBits);
     // complete the register loads: the DMAs below are invisible to the compiler
     fta_wait_vmcnt<0>();
 
@@ -1927,11 +1929,11 @@ __global__ __launch_bounds__(256, DkvSplitShape<D>::WPC) void fta_sparse_dkv_spl
             l_base = l_isd ? dlp : lsep;
             if (gq > 0) {
                 __syncthreads();  // the previous head's membership rows are no longer read
-                bits_lds = fta_stage_kv_bits<TT>(a, bh, wk, Tb, sBits);
+                bits_lds = fta_stage_kv_bits<1>(a, bh, wk, 1, sBits);
             }
             for (int seg0 = 0; seg0 < a.NC; seg0 += SEG) {
                 const int segn = min(SEG, a.NC - seg0);
-                const int Ua = fta_build_kv_masks<TT, SEG>(a, bh, wk, Tb, seg0, segn, bits_lds, sBits, sMask, sList, s_tmp);
+                const int Ua = fta_build_kv_masks<1, SEG>(a, bh, wk, 1, seg0, segn, bits_lds, sBits, sMask, sList, s_tmp);
                 // this part's chunk-list positions [u_lo, u_lo + U) (workgroup-uniform)
                 int u_lo = 0, U = Ua;
                 if constexpr (SPLIT) {
@@ -1981,7 +1983,7 @@ __global__ __launch_bounds__(256, DkvSplitShape<D>::WPC) void fta_sparse_dkv_spl
                 // repeat its last chunk, so every step issues the same number.
                 const int last = U - 1;
                 int c1 = __builtin_amdgcn_readfirstlane((int)lst[0]);
-                uint32_t mk = __builtin_amdgcn_readfirstlane(sMask[tt][c1]), mkp = 0u;
+                uint32_t mk = __builtin_amdgcn_readfirstlane(sMask[0][c1]), mkp = 0u;
                 issue(0, 2, seg0 + c1, seg0 + c1);
                 int c2 = __builtin_amdgcn_readfirstlane((int)lst[min(1, last)]);
                 issue(1, 0, seg0 + c2, seg0 + c1);
@@ -1998,7 +2000,7 @@ __global__ __launch_bounds__(256, DkvSplitShape<D>::WPC) void fta_sparse_dkv_spl
                     // Q_k, dO_{k-1} and P_{k-1} visible; the slots of Q_{k-2}, dO_{k-2} and sX[k & 1] free
                     __syncthreads();
                     issue(k + 2, ds == 0 ? 2 : ds - 1, seg0 + c2, seg0 + c1);
-                    const uint32_t v_mk = sMask[tt][c1];
+                    const uint32_t v_mk = sMask[0][c1];
                     const int v_c = lst[min(k + 3, last)];
                     const float* ld = &sL[k & 3][0];
                     const uint32_t dbase = ldd + ds * TILE_B;

@@ -149,3 +149,56 @@ def test_wide_query_blocks(N, H, D, g):
            for tm, gg, qp in ((fine, 64, q64), (lists, g, qpad))]
     for x, y in zip(*res):
         assert torch.equal(x, y)
+
+
+# chunks (32 queries) that select each KV block: none, single ones at both ends, the last
+# of a mask segment of 1024 and the first of the next, runs of every length up to 7
+CHUNK_SETS = [[], [0], [1249], [5, 1023], [1023, 1024], [0, 1, 2], [7, 8, 1024, 1249], list(range(1021, 1028)),
+              [3, 4, 5, 6, 7], list(range(30, 36)), [1024], list(range(100, 133))]
+
+
+@pytest.mark.parametrize("D,H,Hk,dt", [(64, 1, 1, torch.bfloat16), (128, 1, 1, torch.float16), (256, 1, 1, torch.bfloat16),
+                                       (64, 3, 1, torch.float16), (128, 4, 2, torch.bfloat16)])
+def test_dkv_chunk_lists(D, H, Hk, dt):
+    """dK / dV walks of 0 to 33 chunks in one and two mask segments (1250 chunks), against
+    float64.  P and dS are rounded to 16 bits once (relative error u = 2^-9 or 2^-12) and so
+    are o, which delta is formed from, and the results; every bound below allows 2 u."""
+    N, g, b, W = 40000, 32, 64, 4
+    say(f"[chunk lists] D{D} H{H}/{Hk}")
+    u2 = 2.0**-8 if dt == torch.bfloat16 else 2.0**-11
+    QM, M, G, scale = N // g, N // b, H // Hk, D ** -0.5
+    lists = torch.full((1, H, QM, W), -1, dtype=torch.int32)
+    for h in range(H):
+        for i, chunks in enumerate(CHUNK_SETS):
+            m = (53 * i + 17 * h) % M
+            for c in chunks:
+                c = min(c + 2 * h, QM - 1)
+                row = lists[0, h, c]
+                if m not in row.tolist():
+                    row[(row >= 0).sum()] = m
+    q, do = (rand((1, N, H * D), 70 + i, dt, "cuda") for i in range(2))
+    k, v = (rand((1, N, Hk * D), 72 + i, dt, "cuda") for i in range(2))
+    ql, kl, vl = (x.detach().requires_grad_(True) for x in (q, k, v))
+    o, lse = fta.flash_topk_attn(ql, kl, vl, lists.cuda(), None, H, g, b, num_kv_heads=Hk)
+    got = [x.double().cpu()[0].view(N, -1, D) for x in torch.autograd.grad(o, (ql, kl, vl), do)]
+    q, k, v, do = (x.double().cpu()[0].view(N, -1, D) for x in (q, k, v, do))
+    ref, tol = ([torch.zeros_like(x) for x in (q, k, v)] for _ in range(2))
+    for h in range(H):
+        for c in range(QM):
+            ids = [m for m in lists[0, h, c].tolist() if m >= 0]
+            if not ids:
+                continue
+            r, s = slice(c * g, c * g + g), torch.cat([torch.arange(m * b, m * b + b) for m in ids])
+            Q, K, V, O = q[r, h], k[s, h // G], v[s, h // G], do[r, h]
+            P = (Q @ K.T * scale).softmax(-1)
+            o64 = P @ V
+            dS = P * (O @ V.T - (o64 * O).sum(-1, keepdim=True))
+            dSt = u2 * dS.abs() + u2 * P * (o64 * O).abs().sum(-1, keepdim=True)  # rounded dS, delta from rounded o
+            ref[0][r, h] += dS @ K * scale
+            tol[0][r, h] += dSt @ K.abs() * scale
+            ref[1][s, h // G] += dS.T @ Q * scale
+            tol[1][s, h // G] += dSt.T @ Q.abs() * scale
+            ref[2][s, h // G] += P.T @ O
+            tol[2][s, h // G] += u2 * P.T @ O.abs()
+    for name, x, y, t in zip(("dq", "dk", "dv"), got, ref, tol):
+        assert ((x - y).abs() <= t + u2 * y.abs()).all(), name
