@@ -63,6 +63,9 @@ struct AttnArgs {
     const float* lse2_in;   // lse_in * log2(e), [BH][N] (workspace; dK/dV split kernel)
     const float* delta_in;  // backward input
     int H, N, Dreal, g, kvb, q_pad, kv_pad, Mkv, NC;
+    // end of the rows that the pipelined kernels gather by 32-bit lane offsets: N, or 0
+    // for token strides that these cannot span (every row by a 64-bit address)
+    int q_lim, d_lim, kv_lim;
     int Hk, G;  // K/V heads and query heads per K/V head (G = H / Hk; 1 without GQA)
     float c, scale;
     int wg_per_bh, total;
@@ -522,7 +525,8 @@ __device__ __forceinline__ void fta_compact_masks(uint32_t* row, const uint16_t*
 
 // Gathers the 64 K and V rows at padded key offset kb (the chunk's first row,
 // relative to the sequence) into the stage at LDS address sb: one SGPR base per
-// tensor and a 32-bit byte offset per lane.  Rows outside [0, N) are clamped
+// tensor and a 32-bit byte offset per lane where the caller says that the rows are
+// inside [0, kv_lim), else a 64-bit address per lane, with rows outside [0, N) clamped
 // into it (masked by the caller).
 template <int D, int NW>
 __device__ __forceinline__ void fta_gather_kv(const AttnArgs& a, const uint16_t* kp, const uint16_t* vp, int kb,
@@ -530,24 +534,26 @@ __device__ __forceinline__ void fta_gather_kv(const AttnArgs& a, const uint16_t*
                                               int wave, int lane) {
     using Sh = FwdPipeShape<D, NW>;
     using SW = FtaSwz<Sh::QSEG>;
-    const int t0 = min(max(kb, 0), a.N - 1);
-    const uint16_t* kbp = kp + (int64_t)t0 * a.k_sn;
-    const uint16_t* vbp = vp + (int64_t)t0 * a.v_sn;
     if (inside) {
+        const uint16_t* kbp = kp + (int64_t)kb * a.k_sn;
+        const uint16_t* vbp = vp + (int64_t)kb * a.v_sn;
 #pragma unroll
         for (int i = 0; i < Sh::LQ; ++i) fta_dma16_so(kbp, koff[i], sb + (i * NW + wave) * 1024);
 #pragma unroll
         for (int i = 0; i < Sh::LQ; ++i) fta_dma16_so(vbp, voff[i], sb + Sh::TEN_B + (i * NW + wave) * 1024);
     } else {
+        // addresses formed here, not kept live across the chunk loop for this rare case
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
 #pragma unroll
         for (int i = 0; i < Sh::LQ; ++i) {
-            const int sidx = (i * NW + wave) * 64 + lane;
+            const int sidx = (i * NW + wave) * 64 + ln;
             const int row = sidx / Sh::QSEG;
             int j = SW::slot(row, sidx - row * Sh::QSEG);
             if (j * 8 >= a.Dreal) j = 0;
-            const uint32_t rel = (uint32_t)(min(max(kb + row, 0), a.N - 1) - t0);  // 0 .. 63
-            fta_dma16_so(kbp, 2u * (rel * (uint32_t)a.k_sn + j * 8), sb + (i * NW + wave) * 1024);
-            fta_dma16_so(vbp, 2u * (rel * (uint32_t)a.v_sn + j * 8), sb + Sh::TEN_B + (i * NW + wave) * 1024);
+            const int64_t t = min(max(kb + row, 0), a.N - 1);
+            fta_dma16_at(kp + t * a.k_sn + j * 8, sb + (i * NW + wave) * 1024);
+            fta_dma16_at(vp + t * a.v_sn + j * 8, sb + Sh::TEN_B + (i * NW + wave) * 1024);
         }
     }
 }
@@ -661,7 +667,7 @@ __global__ __launch_bounds__(NW * 64, D <= 64 ? 4 : 1) void fta_sparse_fwd_pipe_
         // gather the walk's next chunk into stage buffer st
         auto issue = [&](int st) {
             const int kb = (seg0 + w.im) * a.kvb - a.kv_pad + w.ich * 64;
-            const bool inside = kb >= 0 && kb + 64 <= a.N && a.kvb - w.ich * 64 >= 64;
+            const bool inside = kb >= 0 && kb + 64 <= a.kv_lim && a.kvb - w.ich * 64 >= 64;
             fta_gather_kv<D, NW>(a, kp, vp, kb, inside, koff, voff, lds0 + st * Sh::STAGE_B, wave, lane);
             w.next_gather();
         };
@@ -1185,7 +1191,7 @@ __global__ __launch_bounds__(512, 1) void fta_sparse_dq_pipe_kernel(AttnArgs a) 
         // gather the walk's next chunk into stage buffer st
         auto issue = [&](int st) {
             const int kb = (seg0 + w.im) * a.kvb - a.kv_pad + w.ich * 64;
-            const bool inside = kb >= 0 && kb + 64 <= a.N && a.kvb - w.ich * 64 >= 64;
+            const bool inside = kb >= 0 && kb + 64 <= a.kv_lim && a.kvb - w.ich * 64 >= 64;
             fta_gather_kv<D, NW>(a, kp, vp, kb, inside, koff, voff, lds0 + st * Sh::STAGE_B, wave, lane);
             w.next_gather();
         };
@@ -1882,7 +1888,7 @@ __global__ __launch_bounds__(256, DkvSplitShape<D>::WPC) void fta_sparse_dkv_spl
     fta_wait_vmcnt<0>();
 
     // Per-lane DMA sources: instruction i of this wave fills 1 KB block i * NW + wave
-    // of a Q or dO tile; qoff / doff = row * stride + column, in bytes (strides <= 2^24)
+    // of a Q or dO tile; qoff / doff = row * stride + column, in bytes (used up to q_lim / d_lim)
     uint32_t qoff[LQ], doff[LQ];
 #pragma unroll
     for (int i = 0; i < LQ; ++i) {
@@ -1945,31 +1951,32 @@ __global__ __launch_bounds__(256, DkvSplitShape<D>::WPC) void fta_sparse_dkv_spl
                 const uint16_t* lst = sList + u_lo;
 
                 // gather one tile of a tensor: chunk c's 32 rows to LDS address lds
-                auto tile = [&](const uint16_t* base, int64_t sn, const uint32_t* off, int c, uint32_t lds)
+                auto tile = [&](const uint16_t* base, int64_t sn, int lim, const uint32_t* off, int c, uint32_t lds)
                     __attribute__((always_inline)) {
                     const int t0 = 32 * c - a.q_pad;
-                    const int tb = min(max(t0, 0), a.N - 1);
-                    const uint16_t* bp = base + (int64_t)tb * sn;
-                    if (t0 >= 0 && t0 + 31 < a.N) {
+                    if (t0 >= 0 && t0 + 31 < lim) {
+                        const uint16_t* bp = base + (int64_t)t0 * sn;
 #pragma unroll
                         for (int i = 0; i < LQ; ++i) fta_dma16_so(bp, off[i], lds + (i * NW + wave) * 1024);
-                    } else {  // a chunk at a sequence edge: clamp its rows (masked off) into [0, N)
+                    } else {  // 64-bit addresses; a chunk at a sequence edge clamps its rows (masked off) into [0, N)
+                        int ln = lane;  // nothing of this rare case is kept live across the steps
+                        asm volatile("" : "+v"(ln));
 #pragma unroll
                         for (int i = 0; i < LQ; ++i) {
-                            const int r2 = (i * NW + wave) * 64 + lane;
+                            const int r2 = (i * NW + wave) * 64 + ln;
                             const int row = r2 / QSEG;
                             int j = SW::slot(row, r2 - row * QSEG);
                             if (j * 8 >= a.Dreal) j = 0;
-                            const uint32_t rel = (uint32_t)(min(max(t0 + row, 0), a.N - 1) - tb);  // 0 .. 31
-                            fta_dma16_so(bp, 2u * (rel * (uint32_t)sn + j * 8), lds + (i * NW + wave) * 1024);
+                            const int64_t t = min(max(t0 + row, 0), a.N - 1);
+                            fta_dma16_at(base + t * sn + j * 8, lds + (i * NW + wave) * 1024);
                         }
                     }
                 };
                 // step kq - 2's gathers: Q and lse of chunk cq (list entry kq), dO and delta
                 // of chunk cd (entry kq - 1)
                 auto issue = [&](int kq, int dslot, int cq, int cd) __attribute__((always_inline)) {
-                    tile(qp, a.q_sn, qoff, cq, ldq + (kq & 3) * TILE_B);
-                    tile(dp, a.d_sn, doff, cd, ldd + dslot * TILE_B);
+                    tile(qp, a.q_sn, a.q_lim, qoff, cq, ldq + (kq & 3) * TILE_B);
+                    tile(dp, a.d_sn, a.d_lim, doff, cd, ldd + dslot * TILE_B);
                     if (wave == 0) {
                         const int t = min(max(32 * (l_isd ? cd : cq) - a.q_pad + l_row, 0), a.N - 1);
                         fta_dma4_at(l_base + t, ldl + (kq & 3) * 256);
@@ -2238,6 +2245,10 @@ int geometry(int B, int H, int N, int D, int g, int kvb, int qph, int qpt, int k
     return FTA_OK;
 }
 
+// Token strides whose byte offsets over a 64-row tile fit the 32-bit lane offsets of
+// the gathers (64 * 2^24 * 2 bytes = 2^31); rows of others are gathered by 64-bit addresses.
+bool narrow_stride(int64_t sn) { return sn >= 0 && sn <= (1 << 24); }
+
 void fill_common(AttnArgs& a, int H, int N, int D, int g, int kvb, int qph, int kvph, float scale, const Geo& G) {
     a.H = H;
     a.Hk = H;  // no GQA unless the caller sets Hk / G
@@ -2254,16 +2265,13 @@ void fill_common(AttnArgs& a, int H, int N, int D, int g, int kvb, int qph, int 
     a.QW = (G.QM + 31) / 32;
     a.scale = scale;
     a.c = scale * 1.4426950408889634f;
+    a.q_lim = narrow_stride(a.q_sn) ? N : 0;
+    a.d_lim = narrow_stride(a.d_sn) ? N : 0;
+    a.kv_lim = narrow_stride(a.k_sn) && narrow_stride(a.v_sn) ? N : 0;
 }
-
-// Token strides whose byte offsets over a 64-row tile fit the 32-bit lane offsets of
-// the gathers (64 * 2^24 * 2 bytes = 2^31); others run on the register-staged kernels.
-bool narrow_stride(int64_t sn) { return sn >= 0 && sn <= (1 << 24); }
 
 template <int DT>
 int launch_fwd_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
-    // the pipelined kernel keeps per-lane row offsets (64 rows x stride) in 32 bits
-    const bool pipe_ok = narrow_stride(a.k_sn) && narrow_stride(a.v_sn);
     switch (Dk) {
 #define FTA_FWD(DK, TPW, NW)                                                                              \
     case DK:                                                                                              \
@@ -2271,21 +2279,17 @@ int launch_fwd_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
         break;
         FTA_FWD(32, 1, 8)
         case 64:
-            if (pipe_ok && a.nsplit > 1)
+            if (a.nsplit > 1)
                 hipLaunchKernelGGL((fta_sparse_fwd_pipe_kernel<DT, 64, 8, true>), dim3(grid), dim3(512), 0, st, a);
-            else if (pipe_ok)
-                hipLaunchKernelGGL((fta_sparse_fwd_pipe_kernel<DT, 64, 8, false>), dim3(grid), dim3(512), 0, st, a);
             else
-                hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, 64, 1, 8, false>), dim3(grid), dim3(512), 0, st, a);
+                hipLaunchKernelGGL((fta_sparse_fwd_pipe_kernel<DT, 64, 8, false>), dim3(grid), dim3(512), 0, st, a);
             break;
         FTA_FWD(96, 1, 8)
         case 128:
-            if (pipe_ok && a.nsplit > 1)
+            if (a.nsplit > 1)
                 hipLaunchKernelGGL((fta_sparse_fwd_pipe_kernel<DT, 128, 8, true>), dim3(grid), dim3(512), 0, st, a);
-            else if (pipe_ok)
-                hipLaunchKernelGGL((fta_sparse_fwd_pipe_kernel<DT, 128, 8, false>), dim3(grid), dim3(512), 0, st, a);
             else
-                hipLaunchKernelGGL((fta_sparse_fwd_kernel<DT, 128, 1, 8, false>), dim3(grid), dim3(512), 0, st, a);
+                hipLaunchKernelGGL((fta_sparse_fwd_pipe_kernel<DT, 128, 8, false>), dim3(grid), dim3(512), 0, st, a);
             break;
         FTA_FWD(160, 1, 8)
         case 256:
@@ -2312,12 +2316,10 @@ int launch_fwd_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
 
 template <int DT>
 int launch_dq_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
-    // the pipelined kernel keeps per-lane row offsets (64 rows x stride) in 32 bits
-    const bool pipe_ok = narrow_stride(a.k_sn) && narrow_stride(a.v_sn);
     // split walks (decided by the caller, grid included): the pipelined kernels (D 64 /
     // 128) or the register-staged ones (D 160 / 256)
     const bool split = a.nsplit > 1;
-    if (split && !(Dk == 160 || Dk == 256 || ((Dk == 64 || Dk == 128) && pipe_ok)))
+    if (split && !(Dk == 64 || Dk == 128 || Dk == 160 || Dk == 256))
         return fta::arg_error("sparse_attn_bwd: no split dQ kernel for this shape");
     switch (Dk) {
 #define FTA_DQ(DK, NW)                                                                                  \
@@ -2333,10 +2335,8 @@ int launch_dq_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
         case 64:
             if (split)
                 hipLaunchKernelGGL((fta_sparse_dq_pipe_kernel<DT, 64, true>), dim3(grid), dim3(512), 0, st, a);
-            else if (pipe_ok)
-                hipLaunchKernelGGL((fta_sparse_dq_pipe_kernel<DT, 64, false>), dim3(grid), dim3(512), 0, st, a);
             else
-                hipLaunchKernelGGL((fta_sparse_dq_kernel<DT, 64, 8, false>), dim3(grid), dim3(512), 0, st, a);
+                hipLaunchKernelGGL((fta_sparse_dq_pipe_kernel<DT, 64, false>), dim3(grid), dim3(512), 0, st, a);
             break;
         case 96:
             hipLaunchKernelGGL((fta_sparse_dq_kernel<DT, 96, 8, false>), dim3(grid), dim3(512), 0, st, a);
@@ -2344,10 +2344,8 @@ int launch_dq_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
         case 128:
             if (split)
                 hipLaunchKernelGGL((fta_sparse_dq_pipe_kernel<DT, 128, true>), dim3(grid), dim3(512), 0, st, a);
-            else if (pipe_ok)
-                hipLaunchKernelGGL((fta_sparse_dq_pipe_kernel<DT, 128, false>), dim3(grid), dim3(512), 0, st, a);
             else
-                hipLaunchKernelGGL((fta_sparse_dq_kernel<DT, 128, 8, false>), dim3(grid), dim3(512), 0, st, a);
+                hipLaunchKernelGGL((fta_sparse_dq_pipe_kernel<DT, 128, false>), dim3(grid), dim3(512), 0, st, a);
             break;
         FTA_DQ(160, 4)
         FTA_DQ(256, 4)
@@ -2375,8 +2373,6 @@ int launch_dq_dt(AttnArgs& a, int Dk, int grid, hipStream_t st) {
 template <int DT>
 int launch_dkv_dt(AttnArgs& a, int Dk, int Tb, int B, int H, int ntiles, hipStream_t st) {
     const bool gqa = a.G > 1;
-    // the split kernel keeps per-lane Q / dO row offsets in 32 bits
-    const bool split_ok = Tb == 2 && narrow_stride(a.q_sn) && narrow_stride(a.d_sn);
     // ns: parts per KV block (the split kernel with a.nsplit > 1), else 1
     auto go = [&](auto kern, int tt, int nw, int ns) {
         a.wg_per_bh = (ntiles + tt - 1) / tt;
@@ -2405,7 +2401,7 @@ int launch_dkv_dt(AttnArgs& a, int Dk, int Tb, int B, int H, int ntiles, hipStre
             : go(fta_sparse_dkv_split_kernel<DT, DK, false, false>, 2, 4, 1)
         FTA_DKV(32, 8, 1, 4, 2, 4)
         case 64:
-            if (split_ok)
+            if (Tb == 2)
                 FTA_DKV_SPLIT(64);
             else if (Tb == 1)
                 FTA_DKV_GO(64, 1, 4);
@@ -2414,7 +2410,7 @@ int launch_dkv_dt(AttnArgs& a, int Dk, int Tb, int B, int H, int ntiles, hipStre
             break;
         FTA_DKV(96, 4, 1, 4, 2, 2)
         case 128:
-            if (split_ok)
+            if (Tb == 2)
                 FTA_DKV_SPLIT(128);
             else if (Tb == 1)
                 FTA_DKV_GO(128, 1, 4);
@@ -2423,7 +2419,7 @@ int launch_dkv_dt(AttnArgs& a, int Dk, int Tb, int B, int H, int ntiles, hipStre
             break;
         FTA_DKV(160, 4, 2, 2, 2, 2)
         case 256:
-            if (split_ok)
+            if (Tb == 2)
                 FTA_DKV_SPLIT(256);
             else
                 FTA_DKV_GO(256, 4, 1);
@@ -2601,8 +2597,7 @@ int fta_sparse_attn_fwd_gqa(const void* q, const int64_t* q_strides, const void*
     // split walks (small grids, workspace for the parts)
     const int ns = fwd_nsplit(B, H, G);
     const bool split = ns > 1 && workspace != nullptr &&
-                       workspace_bytes >= fwd_bytes(B, H) + split_bytes(B, H, G, ns) &&
-                       (G.Dk > 128 || (narrow_stride(k_strides[2]) && narrow_stride(v_strides[2])));
+                       workspace_bytes >= fwd_bytes(B, H) + split_bytes(B, H, G, ns);
     a.nsplit = split ? ns : 1;
     a.nbh = B * H;
     a.npq = G.Npq;
@@ -2723,9 +2718,7 @@ int bwd_dq_impl(const int32_t* head_perm, const void* q, const int64_t* q_stride
     a.wg_per_bh = (G.Npq + 32 * Tq - 1) / (32 * Tq);
     // small grids: each workgroup's union walk in 2-4 parts, summed by fta_dq_combine_kernel
     const int ns = dq_nsplit(B, H, G);
-    const bool pipe_ok = narrow_stride(a.k_sn) && narrow_stride(a.v_sn);
-    const bool split = ns > 1 && (G.Dk > 128 || pipe_ok) && split_ws != nullptr &&
-                       split_avail >= dq_split_bytes(B, H, G, ns);
+    const bool split = ns > 1 && split_ws != nullptr && split_avail >= dq_split_bytes(B, H, G, ns);
     a.nsplit = split ? ns : 1;
     a.nbh = B * H;
     a.npq = G.Npq;
@@ -2802,8 +2795,7 @@ int fta_sparse_attn_bwd_dkv(const void* q, const int64_t* q_strides, const void*
     // fta_dkv_combine_kernel, when the workspace has room for the parts
     const int ns = dkv_nsplit(B, Hk, kv_block_size, G);
     const size_t used = bwd_bytes(B, H, N, G);
-    const bool split = ns > 1 && workspace_bytes >= used + dkv_split_bytes(B, Hk, G, ns) &&
-                       narrow_stride(a.q_sn) && narrow_stride(a.d_sn);
+    const bool split = ns > 1 && workspace_bytes >= used + dkv_split_bytes(B, Hk, G, ns);
     a.nsplit = split ? ns : 1;
     a.nbh = B * Hk;
     a.npq = G.Mkv * 64;

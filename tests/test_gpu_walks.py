@@ -1,6 +1,6 @@
 """Edges of the pipelined attention walks: blocks of several chunks, lists of one
 block, tiles that skip blocks of their workgroup's union, unsplit grids, and
-token strides past the gathers' 32-bit lane offsets."""
+token strides past the gathers' 32-bit lane offsets or below zero."""
 
 import numpy as np
 import pytest
@@ -42,8 +42,8 @@ def test_walk_edges(case):
 
 @pytest.mark.parametrize("D,b", [(64, 64), (128, 64), (256, 64)])
 def test_wide_token_strides(D, b):
-    """Rows 2^24 + 8 elements apart run on the register-staged kernels; the same sums,
-    so o and the gradients are within one bf16 rounding step of the contiguous call."""
+    """Rows 2^24 + 8 elements apart (gathered by 64-bit addresses), one KV block: o and the
+    gradients are within one bf16 rounding step of the contiguous call."""
     N, H, g, W = 40, 1, 16, 1
     say(f"[wide strides] D{D}")
     stride = 2**24 + 8
@@ -64,6 +64,60 @@ def test_wide_token_strides(D, b):
         x, y = x.float().cpu().numpy(), y.float().cpu().numpy()
         step = np.maximum(np.abs(x), np.abs(y)) * 2.0**-7 + np.abs(x).max() * 2.0**-16
         assert (np.abs(x - y) <= step).all(), name
+
+
+@pytest.mark.parametrize("D,b,N,H,Hk,step", [
+    (64, 64, 1000, 2, 2, -1), (128, 64, 1000, 4, 2, -1), (256, 64, 500, 2, 2, -1), (128, 48, 500, 2, 2, -1),
+    (96, 128, 700, 2, 1, -1), (64, 64, 136, 1, 1, 2**24 + 8), (128, 64, 136, 1, 1, 2**24 + 8)])
+def test_token_strides(D, b, N, H, Hk, step):
+    """Tokens stored last to first (negative token strides, C entry) or 2^24 + 8 elements
+    apart, over several KV blocks: the kernels and the order of their sums are those of the
+    contiguous call, so the results are its bits."""
+    from flash_topk_attn_v2 import _lib
+
+    g, dt = 16, torch.bfloat16
+    say(f"[token strides] D{D} b{b} N{N} H{H}/{Hk} step {step}")
+    qpad, kvpad = -N % g, -N % b
+    QM, M = (N + qpad) // g, (N + kvpad) // b
+    merged = torch.from_numpy(_random_merged(1, H, QM, 2, M, 17)).cuda()
+    toks = [rand((N, h * D), 40 + i, dt, "cuda") for i, h in enumerate((H, Hk, Hk, H))]  # q, k, v, do
+    L, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    geo = (g, b, 0, qpad, 0, kvpad)
+
+    def call(views):
+        """o, lse, dq, dk, dv of tokens at (pointer, strides)"""
+        o, dq = (torch.empty(N, H * D, device="cuda", dtype=dt) for _ in range(2))
+        dk, dv = (torch.empty(N, Hk * D, device="cuda", dtype=dt) for _ in range(2))
+        lse = torch.empty(1, H, N, device="cuda")
+        so, sk = _lib.i64arr((N * H * D, D, H * D)), _lib.i64arr((N * Hk * D, D, Hk * D))
+        (q, qs), (k, ks), (v, vs), (do, ds) = views
+        code = _lib.dtype_code(dt)
+        size = (1, H, N, D, *geo)
+        ws = torch.empty(max(L.fta_sparse_attn_fwd_workspace_size(*size), L.fta_sparse_attn_bwd_workspace_size(*size)),
+                         dtype=torch.uint8, device="cuda")
+        shape = (1, H, Hk, N, D, merged.data_ptr(), QM, 2, *geo, D ** -0.5)
+        _lib.check(L.fta_sparse_attn_fwd_gqa(q, qs, k, ks, v, vs, code, *shape, o.data_ptr(), so, lse.data_ptr(),
+                                             ws.data_ptr(), ws.numel(), stream), "fwd")
+        delta = (o.float() * toks[3].float()).view(N, H, D).sum(-1).T.contiguous()
+        _lib.check(L.fta_sparse_attn_bwd_gqa(q, qs, k, ks, v, vs, do, ds, code, *shape, lse.data_ptr(),
+                                             delta.data_ptr(), dq.data_ptr(), so, dk.data_ptr(), sk, dv.data_ptr(), sk,
+                                             ws.data_ptr(), ws.numel(), stream), "bwd")
+        torch.cuda.synchronize()
+        return o, lse, dq, dk, dv
+
+    want = call([(t.data_ptr(), _lib.i64arr((t.numel(), D, t.shape[1]))) for t in toks])
+    keep, views = [], []
+    for t in toks:
+        if step < 0:
+            store = t.flip(0).contiguous()
+            views.append((store[-1].data_ptr(), _lib.i64arr((t.numel(), D, -t.shape[1]))))
+        else:
+            store = torch.empty((N - 1) * step + t.shape[1], dtype=dt, device="cuda")
+            store.as_strided(t.shape, (step, 1)).copy_(t)
+            views.append((store.data_ptr(), _lib.i64arr((N * step, D, step))))
+        keep.append(store)
+    for name, x, y in zip(("o", "lse", "dq", "dk", "dv"), want, call(views)):
+        assert torch.equal(x, y), name
 
 
 @pytest.mark.parametrize("W,offset", [(5, 0), (8, 0), (8, 1), (12, 2), (1, 3)])
