@@ -2561,9 +2561,10 @@ int fta_sparse_attn_fwd_gqa(const void* q, const int64_t* q_strides, const void*
     const int T = (G.Dk <= 160) ? 8 : 4;  // query tiles per workgroup
     const int64_t wgs = (int64_t)((G.Npq + 32 * T - 1) / (32 * T)) * B * H;
     // XCD placement of the heads by their work (only with a workspace: callers
-    // that pass none keep the natural order; and only when the workgroups do not
-    // all run at once, one per CU, where the placement cannot change the time)
-    if (workspace != nullptr && workspace_bytes >= fwd_bytes(B, H) && wgs > 256) {
+    // that pass none keep the natural order; only when the workgroups do not
+    // all run at once, one per CU, where the placement cannot change the time;
+    // and only for the pipelined kernels, which read it)
+    if (G.Dk <= 128 && workspace != nullptr && workspace_bytes >= fwd_bytes(B, H) && wgs > 256) {
         int32_t* head_work = (int32_t*)workspace;
         int32_t* head_perm = head_work + B * H;
         if ((rc = fta::launch_head_order_merged(merged_indices, B * H, QM, W, G.Mkv, max(1, 256 / q_block_size), head_work, head_perm, st)) !=

@@ -120,6 +120,30 @@ def test_token_strides(D, b, N, H, Hk, step):
         assert torch.equal(x, y), name
 
 
+@pytest.mark.parametrize("D,H", [(160, 66), (256, 33)])
+def test_wide_heads_leave_workspace(D, H):
+    """Forwards of wide heads with more than 256 workgroups use no head placement and no
+    split: nothing is computed into the workspace."""
+    from flash_topk_attn_v2 import _lib
+
+    N, g, b = 1024, 64, 64
+    say(f"[workspace] D{D} H{H}")
+    merged = torch.from_numpy(_random_merged(1, H, N // g, 2, N // b, 19)).cuda()
+    q, k, v = (rand((1, N, H * D), 80 + i, torch.float16, "cuda") for i in range(3))
+    want = fta.flash_topk_attn(q, k, v, merged, None, H, g, b)[0]
+    L, st = _lib.lib(), _lib.i64arr((N * H * D, D, H * D))
+    nbytes = L.fta_sparse_attn_fwd_workspace_size(1, H, N, D, g, b, 0, 0, 0, 0)
+    ws = torch.full((nbytes,), 0x5A, dtype=torch.uint8, device="cuda")
+    o, lse = torch.empty_like(want), torch.empty(1, H, N, device="cuda")
+    _lib.check(L.fta_sparse_attn_fwd_gqa(q.data_ptr(), st, k.data_ptr(), st, v.data_ptr(), st, _lib.dtype_code(q.dtype),
+                                         1, H, H, N, D, merged.data_ptr(), N // g, 2, g, b, 0, 0, 0, 0, D ** -0.5,
+                                         o.data_ptr(), st, lse.data_ptr(), ws.data_ptr(), nbytes,
+                                         torch.cuda.current_stream().cuda_stream), "fta_sparse_attn_fwd_gqa")
+    torch.cuda.synchronize()
+    assert torch.equal(o, want)
+    assert bool((ws == 0x5A).all())
+
+
 @pytest.mark.parametrize("W,offset", [(5, 0), (8, 0), (8, 1), (12, 2), (1, 3)])
 def test_list_loads(W, offset):
     """Merged lists are read 16 bytes at a time where a row is a multiple of 4 ids on a
