@@ -229,40 +229,16 @@ def test_wide_query_blocks(N, H, D, g):
         assert torch.equal(x, y)
 
 
-# chunks (32 queries) that select each KV block: none, single ones at both ends, the last
-# of a mask segment of 1024 and the first of the next, runs of every length up to 7
-CHUNK_SETS = [[], [0], [1249], [5, 1023], [1023, 1024], [0, 1, 2], [7, 8, 1024, 1249], list(range(1021, 1028)),
-              [3, 4, 5, 6, 7], list(range(30, 36)), [1024], list(range(100, 133))]
-
-
-@pytest.mark.parametrize("D,H,Hk,dt", [(64, 1, 1, torch.bfloat16), (128, 1, 1, torch.float16), (256, 1, 1, torch.bfloat16),
-                                       (64, 3, 1, torch.float16), (128, 4, 2, torch.bfloat16)])
-def test_dkv_chunk_lists(D, H, Hk, dt):
-    """dK / dV walks of 0 to 33 chunks in one and two mask segments (1250 chunks), against
-    float64.  P and dS are rounded to 16 bits once (relative error u = 2^-9 or 2^-12) and so
-    are o, which delta is formed from, and the results; every bound below allows 2 u."""
-    N, g, b, W = 40000, 32, 64, 4
-    say(f"[chunk lists] D{D} H{H}/{Hk}")
-    u2 = 2.0**-8 if dt == torch.bfloat16 else 2.0**-11
-    QM, M, G, scale = N // g, N // b, H // Hk, D ** -0.5
-    lists = torch.full((1, H, QM, W), -1, dtype=torch.int32)
-    for h in range(H):
-        for i, chunks in enumerate(CHUNK_SETS):
-            m = (53 * i + 17 * h) % M
-            for c in chunks:
-                c = min(c + 2 * h, QM - 1)
-                row = lists[0, h, c]
-                if m not in row.tolist():
-                    row[(row >= 0).sum()] = m
-    q, do = (rand((1, N, H * D), 70 + i, dt, "cuda") for i in range(2))
-    k, v = (rand((1, N, Hk * D), 72 + i, dt, "cuda") for i in range(2))
-    ql, kl, vl = (x.detach().requires_grad_(True) for x in (q, k, v))
-    o, lse = fta.flash_topk_attn(ql, kl, vl, lists.cuda(), None, H, g, b, num_kv_heads=Hk)
-    got = [x.double().cpu()[0].view(N, -1, D) for x in torch.autograd.grad(o, (ql, kl, vl), do)]
-    q, k, v, do = (x.double().cpu()[0].view(N, -1, D) for x in (q, k, v, do))
+def _check_grads(tokens, lists, got, H, Hk, D, g, b):
+    """dq, dk, dv (``got``) of one unpadded sequence against float64.  P and dS are rounded
+    to 16 bits once (relative error u = 2^-9 or 2^-12) and so are o, which delta is formed
+    from, and the results; every bound allows 2 u."""
+    u2 = 2.0**-8 if tokens[0].dtype == torch.bfloat16 else 2.0**-11
+    N, G, scale = tokens[0].shape[1], H // Hk, D ** -0.5
+    q, k, v, do = (x.detach().double().cpu()[0].view(N, -1, D) for x in tokens)
     ref, tol = ([torch.zeros_like(x) for x in (q, k, v)] for _ in range(2))
     for h in range(H):
-        for c in range(QM):
+        for c in range(N // g):
             ids = [m for m in lists[0, h, c].tolist() if m >= 0]
             if not ids:
                 continue
@@ -279,4 +255,58 @@ def test_dkv_chunk_lists(D, H, Hk, dt):
             ref[2][s, h // G] += P.T @ O
             tol[2][s, h // G] += u2 * P.T @ O.abs()
     for name, x, y, t in zip(("dq", "dk", "dv"), got, ref, tol):
+        x = x.double().cpu()[0].view(N, -1, D)
         assert ((x - y).abs() <= t + u2 * y.abs()).all(), name
+
+
+# chunks (32 queries) that select each KV block: none, single ones at both ends, the last
+# of a mask segment of 1024 and the first of the next, runs of every length up to 7
+CHUNK_SETS = [[], [0], [1249], [5, 1023], [1023, 1024], [0, 1, 2], [7, 8, 1024, 1249], list(range(1021, 1028)),
+              [3, 4, 5, 6, 7], list(range(30, 36)), [1024], list(range(100, 133))]
+
+
+@pytest.mark.parametrize("D,H,Hk,dt", [(64, 1, 1, torch.bfloat16), (128, 1, 1, torch.float16), (256, 1, 1, torch.bfloat16),
+                                       (64, 3, 1, torch.float16), (128, 4, 2, torch.bfloat16)])
+def test_dkv_chunk_lists(D, H, Hk, dt):
+    """dK / dV walks of 0 to 33 chunks in one and two mask segments (1250 chunks)."""
+    N, g, b, W = 40000, 32, 64, 4
+    say(f"[chunk lists] D{D} H{H}/{Hk}")
+    QM, M = N // g, N // b
+    lists = torch.full((1, H, QM, W), -1, dtype=torch.int32)
+    for h in range(H):
+        for i, chunks in enumerate(CHUNK_SETS):
+            m = (53 * i + 17 * h) % M
+            for c in chunks:
+                c = min(c + 2 * h, QM - 1)
+                row = lists[0, h, c]
+                if m not in row.tolist():
+                    row[(row >= 0).sum()] = m
+    q, do = (rand((1, N, H * D), 70 + i, dt, "cuda") for i in range(2))
+    k, v = (rand((1, N, Hk * D), 72 + i, dt, "cuda") for i in range(2))
+    ql, kl, vl = (x.detach().requires_grad_(True) for x in (q, k, v))
+    o, lse = fta.flash_topk_attn(ql, kl, vl, lists.cuda(), None, H, g, b, num_kv_heads=Hk)
+    _check_grads((q, k, v, do), lists, torch.autograd.grad(o, (ql, kl, vl), do), H, Hk, D, g, b)
+
+
+@pytest.mark.parametrize("N,H,Hk,D,g,W", [
+    (6272, 16, 8, 64, 32, 2),  # 784 blocks, 768 run at once; bitmap rows of 7 words
+    (6272, 16, 8, 64, 64, 1),  # rows of 4 words (16-byte loads)
+    (4160, 16, 8, 128, 16, 1),  # 520 blocks, 512 at once; rows of 9 words
+    (2176, 8, 8, 256, 64, 2),  # 272 blocks, 256 at once
+    (2176, 16, 8, 256, 32, 1),
+    (6272, 10, 10, 64, 32, 1),  # heads that no multiple of 8 covers: natural head order
+])
+def test_launch_order(N, H, Hk, D, g, W):
+    """dK / dV grids just above what the chip holds at once, which are launched in the
+    order of the blocks' counts with the heads placed by their work (GQA and D = 256)."""
+    b, dt = 64, torch.bfloat16
+    say(f"[launch order] N{N} H{H}/{Hk} D{D} g{g}")
+    lists = torch.from_numpy(_random_merged(1, H, N // g, W, N // b, 23))
+    lists[:, ::3] %= N // b // 2  # heads of unequal counts per block
+    if W > 1:
+        lists[..., 1] = torch.where(lists[..., 1] == lists[..., 0], -1, lists[..., 1])
+    q, do = (rand((1, N, H * D), 90 + i, dt, "cuda") for i in range(2))
+    k, v = (rand((1, N, Hk * D), 92 + i, dt, "cuda") for i in range(2))
+    ql, kl, vl = (x.detach().requires_grad_(True) for x in (q, k, v))
+    o, lse = fta.flash_topk_attn(ql, kl, vl, lists.cuda(), None, H, g, b, num_kv_heads=Hk)
+    _check_grads((q, k, v, do), lists, torch.autograd.grad(o, (ql, kl, vl), do), H, Hk, D, g, b)
