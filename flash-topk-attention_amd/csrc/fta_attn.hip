@@ -446,7 +446,8 @@ __global__ __launch_bounds__(NW * 64, 1) void fta_sparse_fwd_kernel(AttnArgs a) 
 // scheduling fences: left alone the compiler either keeps a whole chunk's fragments
 // in registers (156 at D = 64) or waits out one LDS latency per MFMA.  B2 N8192 H16
 // D64 fp16, lists of every block: 0.80 -> 0.66 ms; one list of 16 blocks per query:
-// 0.74 -> 0.59-0.62 ms (whole call, with its list preparation); B1 N16384 H16 D128 dense lists: 1.95 -> 1.88 ms.
+// 0.74 -> 0.59-0.62 ms (whole call, with its list preparation); B1 N16384 H16 D128
+// dense lists: 1.95 -> 1.88 ms.
 // ----------------------------------------------------------------------------
 template <int D, int NW>
 struct FwdPipeShape {
@@ -1785,8 +1786,8 @@ __global__ __launch_bounds__(TT * CS * 64, 1) void fta_sparse_dkv_kernel(AttnArg
 // P crosses once, in fp32, so dS is formed from the same fp32 P as with one
 // wave per tile.  Each wave evaluates only its own half of the elementwise work
 // (the exponentials or the dS products), one of K / V and one set of
-// accumulators, so several WGs fit on a CU (three at D = 64, two at D = 128, with
-// registers <= 256 per lane): one WG's mask building and gather latency overlap the
+// accumulators, so several WGs fit on a CU (three at D = 64 with at most 168 registers
+// per lane, two at D = 128 with at most 256): one WG's mask building and gather latency overlap the
 // others' MFMAs.  At D = 256 (twice the tile bytes and accumulators) one WG runs per
 // CU, with the accumulators in the 512-register budget of one wave per SIMD.
 //
@@ -1800,7 +1801,7 @@ __global__ __launch_bounds__(TT * CS * 64, 1) void fta_sparse_dkv_kernel(AttnArg
 // step ahead, P crosses as 16-byte LDS accesses, and the rows a partly selected chunk
 // leaves out are masked with one sign-extended bit each.
 // What bounds it: each chunk's 16 KB (D = 128) serves only 64 keys, so the gathers
-// (7.4 TB/s from L2 on dense lists) and the matrix pipe (40% busy) share the time.
+// (7.4 TB/s from L2 on dense lists) and the matrix pipe (41% busy) share the time.
 // dK/dV on B1 N16384 H16 D128 dense lists 4.41 -> 4.12 ms, B1 N32768 H32 D128 short
 // lists 1.93 -> 1.81 ms, B2 N10000 H12/4 D64 g16 2.23 -> 1.58 ms (most of it from the
 // third WG per CU), N2048 H8 D256 0.118 -> 0.109 ms.
@@ -2452,12 +2453,21 @@ size_t sel_bytes(int B, int H, const Geo& G) {
 // and the 64 partial counts per head they are summed from
 size_t fwd_bytes(int B, int H) { return fta::align_up((size_t)B * H * (2 + 64) * sizeof(int32_t)); }
 
-// Forward parts per workgroup.  A grid of fewer than 128 workgroups (under half
-// the CUs) is bound by each workgroup's sequential union walk, not by the chip:
-// every walk is then split into up to 4 parts (256 / grid) and
-// fta_fwd_combine_kernel merges them.  At D = 256 the workgroups are half as long
-// (128 queries) and 128 of them still leave half the CUs idle: N2048 H8 D256, lists of
-// every block, 139 us unsplit, 81 + 9 us in two parts.  D = 160 is never split.
+// Forward parts per workgroup.  A small grid is bound by each workgroup's
+// sequential union walk, not by the chip: every walk is then split into up to 4
+// parts (256 / grid) and fta_fwd_combine_kernel merges them.  Where the lines lie
+// (whole calls in us, lists of every block / of 4 blocks per 64 queries):
+//  * D = 256 runs one workgroup per CU, so two parts pay up to 128 workgroups, where
+//    all parts run at once, and no further.  96: 73 -> 51 / 41 -> 37; 128: 134 -> 82
+//    (N2048), 73 -> 53 (N1024) / 40 -> 38; 136: 74 -> 91 / 42 -> 58; 240: 136 -> 154 /
+//    43 -> 67.
+//  * D = 64 / 128: below 128 workgroups.  At 128, dense lists gain (D = 128 114 -> 88,
+//    D = 64 88 -> 65 at N4096) and short ones lose (31 -> 34, 24 -> 30), and from 129
+//    both lose (D = 128, 144: 65 -> 89 / 32 -> 50).
+//  * D = 160 is never split.
+// A part rounds P to 16 bits against its own maximum.  o is no further from float64
+// than unsplit (D = 256, N 512 to 4096, both types: 2.34e-3 -> 2.33e-3 at best and
+// 2.12e-3 -> 1.84e-3 at most; dq, dk, dv the same within 0.1% or nearer).
 int fwd_nsplit(int B, int H, const Geo& G) {
     if (!(G.Dk == 64 || G.Dk == 128 || G.Dk == 256) || G.Mkv < 8) return 1;
     const int rows = (G.Dk == 256) ? 128 : 256;  // queries per workgroup
@@ -2494,7 +2504,9 @@ size_t dq_split_bytes(int B, int H, const Geo& G, int ns) {
 int64_t dkv_slots(const Geo& G) { return 256 * ((G.Dk <= 64) ? 3 : (G.Dk <= 128) ? 2 : 1); }
 
 // dK/dV parts of the split kernel (64-key blocks, D 64 / 128 / 256) on small
-// grids: fewer than two workgroups per CU (one at D = 256) get
+// grids: fewer than two workgroups per CU (one at D = 256; at D = 64 three fit, but
+// two parts of 544 to 704 workgroups lose: 704, dense lists 137 -> 151 us, short 60 ->
+// 70) get
 // up to 4 parts per KV block; [dK, dV][part][b * Hk][KV block * 64 + key][Dk]
 // fp32, after bwd_bytes (dQ's parts reuse the same bytes after dK/dV is done)
 int dkv_nsplit(int B, int Hk, int kv_block_size, const Geo& G) {
@@ -2675,7 +2687,7 @@ int bwd_common(AttnArgs& a, Geo& G, const void* q, const int64_t* q_strides, con
 // 64-key blocks at D 64 / 128 / 256 (the split dK/dV kernel) run in the launch
 // order of fta_kv_order_kernel and the head placement of fta_head_balance_kernel,
 // except where all workgroups run at once (the order cannot change the time; the two
-// launches took 10 of 199 us at N2048 H8 D128)
+// launches took 10 of 199 us at N2048 H8 D128, 8 to 10 us at D = 64 and 512 to 768)
 bool uses_kv_order(int B, int Hk, int kv_block_size, const Geo& G) {
     return kv_block_size > 32 && kv_block_size <= 64 && (G.Dk == 64 || G.Dk == 128 || G.Dk == 256) &&
            G.Mkv <= 4096 && (int64_t)G.Mkv * B * Hk > dkv_slots(G);
@@ -2771,7 +2783,7 @@ int fta_sparse_attn_bwd_dkv(const void* q, const int64_t* q_strides, const void*
         return rc;
     a.sel = sel;
     a.lse2_in = lse2;
-    // 64-key blocks at D 64 / 128 (the split kernel): launch in first-q-block order
+    // the split kernel's launch order: KV blocks by selection count, heads by work
     if (uses_kv_order(B, Hk, kv_block_size, G)) {
         int32_t* order = (int32_t*)((char*)lse2 + fta::align_up((size_t)B * H * N * sizeof(float)));
         int32_t* head_work = (int32_t*)((char*)order + fta::align_up((size_t)B * H * G.Mkv * sizeof(int32_t)));

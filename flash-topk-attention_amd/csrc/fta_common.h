@@ -136,8 +136,9 @@ __device__ __forceinline__ uint4 fta_tr_frag(const uint16_t* tile, int row, int 
 //    per C3-iid sparse forward, 5.5e8 per C3 scoring launch);
 //  * ds_read_b64_tr_b16 is served 32 lanes at a time over 256 bytes: 4
 //    consecutive rows x 64 bytes, so bits 2..3 of x must differ across them.
-// x(r) = (r & 3) << 2 | (r >> 2) & 3 meets both for 16 or more slots per row; 8 slots (128-byte rows, two rows per bank line) use the row-pair form; 4
-// slots need none.  12 and 20 slots use r & 3 (not tuned).
+// x(r) = (r & 3) << 2 | (r >> 2) & 3 meets both for 16 or more slots per row; 8
+// slots (128-byte rows, two rows per bank line) use the row-pair form; 4 slots need
+// none.  12 and 20 slots use r & 3 (not tuned).
 // ---------------------------------------------------------------------------
 template <int QSEG>
 struct FtaSwz {

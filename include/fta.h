@@ -98,7 +98,8 @@ int fta_topk_select(const float* block_scores, int64_t rows, int M, int64_t stri
  * Workspace of fta_topk_score.  fta_topk_score_workspace_size covers every
  * path (any head dim, block size and max_topk); fta_topk_score_workspace_size_ex
  * returns the recommended size for one call's geometry (0 for an invalid one),
- * assuming a K token stride of at most 2^24 elements.
+ * assuming a K token stride of 0 to 2^24 elements (other strides store per-block
+ * values: at b = 64 and 128 they need the size that fta_topk_score_workspace_size gives).
  *
  * b = 64 or 128, D <= 128 and at most 32 blocks per query run
  * on candidate streams: chunks of 1024 entries taken from a pool in the
@@ -244,10 +245,11 @@ size_t fta_sparse_attn_fwd_workspace_size(int B, int H, int N, int D, int q_bloc
 /*
  * Parts per workgroup walk of the forward with its workspace for this
  * geometry (0 for an invalid one): 1, or 2-4 when the grid has fewer than 128
- * workgroups and D <= 128, or at most 128 and D > 160.  Then each workgroup's walk over the union of its
- * q-blocks' lists (ascending, per 512-block segment) is split into that many
- * contiguous ranges, each with its own online-softmax anchor, and a combine
- * kernel merges the parts' (O, max, sum).  No counterpart in the reference
+ * workgroups and D <= 128, or at most 128 and D > 160.  Then each workgroup's
+ * walk over the union of its q-blocks' lists (ascending, per 512-block segment)
+ * is split into that many contiguous ranges, each with its own online-softmax
+ * anchor, and a combine kernel merges the parts' (O, max, sum).  No counterpart
+ * in the reference
  * (its forward is never split); exposed so that callers and tests can tell
  * which schedule rounds P.
  */
@@ -306,9 +308,9 @@ int fta_sparse_attn_fwd_gqa(const void* q, const int64_t* q_strides, const void*
  * used by dK/dV and then by dQ): dK/dV with fewer than 512 workgroups (256 at
  * D 256; 64-key blocks at D 64 / 128 / 256) and dQ with fewer than 128
  * workgroups (at most 128 at D 160 / 256) walk their lists in 2-4 parts whose
- * fp32 sums are added by a combine kernel.  A smaller workspace (at least the bitmap, lse and order)
- * runs the walks unsplit: the results then differ only in fp32 summation
- * order.  Sized for Hk = H; with Hk < H the dK/dV parts may not fit, and
+ * fp32 sums are added by a combine kernel.  A smaller workspace (at least the
+ * bitmap, lse and order) runs the walks unsplit: the results then differ only in
+ * fp32 summation order.  Sized for Hk = H; with Hk < H the dK/dV parts may not fit, and
  * dK/dV then runs unsplit.
  */
 size_t fta_sparse_attn_bwd_workspace_size(int B, int H, int N, int D, int q_block_size,
