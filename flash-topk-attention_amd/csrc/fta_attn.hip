@@ -2607,9 +2607,13 @@ int fta_sparse_attn_fwd_gqa(const void* q, const int64_t* q_strides, const void*
     a.Hk = Hk;
     a.G = H / Hk;
     a.wg_per_bh = (G.Npq + 32 * T - 1) / (32 * T);
-    // split walks (small grids, workspace for the parts)
+    // split walks (small grids, workspace for the parts; at D = 256 none of so few chunks
+    // that the parts and their combine cost more than they save: N2048 H8, lists of 2 / 3 /
+    // 4 blocks per 64 queries, 27 / 34 / 41 us unsplit and 31 / 35 / 38 in two parts;
+    // N1024 H8, 27 / 33 / 40 and 27 / 31 / 33 in four)
     const int ns = fwd_nsplit(B, H, G);
-    const bool split = ns > 1 && workspace != nullptr &&
+    const int64_t listed = std::min<int64_t>(G.Mkv, (int64_t)((32 * T + q_block_size - 1) / q_block_size) * W);
+    const bool split = ns > 1 && (G.Dk <= 128 || listed * G.nch > (ns == 2 ? 6 : 4)) && workspace != nullptr &&
                        workspace_bytes >= fwd_bytes(B, H) + split_bytes(B, H, G, ns);
     a.nsplit = split ? ns : 1;
     a.nbh = B * H;

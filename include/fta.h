@@ -245,12 +245,13 @@ size_t fta_sparse_attn_fwd_workspace_size(int B, int H, int N, int D, int q_bloc
 /*
  * Parts per workgroup walk of the forward with its workspace for this
  * geometry (0 for an invalid one): 1, or 2-4 when the grid has fewer than 128
- * workgroups and D <= 128, or at most 128 and D > 160.  Then each workgroup's
- * walk over the union of its q-blocks' lists (ascending, per 512-block segment)
- * is split into that many contiguous ranges, each with its own online-softmax
- * anchor, and a combine kernel merges the parts' (O, max, sum).  No counterpart
- * in the reference
- * (its forward is never split); exposed so that callers and tests can tell
+ * workgroups and D <= 128, or at most 128 and D > 160 (where a call whose
+ * lists are too short runs unsplit all the same: by their width, at most 4
+ * 64-key chunks listed by the q-blocks of 128 queries, 6 where it is 2).  Then
+ * each workgroup's walk over the union of its q-blocks' lists (ascending, per
+ * 512-block segment) is split into that many contiguous ranges, each with its
+ * own online-softmax anchor, and a combine kernel merges the parts' (O, max,
+ * sum).  No counterpart in the reference (its forward is never split); exposed so that callers and tests can tell
  * which schedule rounds P.
  */
 int fta_sparse_attn_fwd_splits(int B, int H, int N, int D, int q_block_size, int kv_block_size,

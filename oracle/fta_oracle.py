@@ -408,8 +408,8 @@ def sparse_attn(
     whenever the maximum grows, as the reference's kernel does,
     v2/csrc/sparse_attn_kernel.cuh:145-160), and the accumulators are scaled by
     2^(c m_old - c m_new) then.  ``splits`` > 1 models this build's split
-    forward (small grids, fta_sparse_attn_fwd_splits): each 256-row workgroup's
-    union walk is cut into that many parts (_split_parts), each part runs the
+    forward (small grids, fta_sparse_attn_fwd_splits): the union walk of each
+    workgroup (256 rows, 128 for D > 160) is cut into that many parts (_split_parts), each part runs the
     schedule above from its own anchor, and the parts are merged as
     o = sum_p acc_p 2^(c m_p - c m) / sum_p l_p 2^(c m_p - c m), m = max m_p."""
     B, N, C = q.shape
@@ -449,11 +449,12 @@ def sparse_attn(
             chunk = _chunk_starts(ids[ids >= 0], N, kv_block_size, kph)
             tok_blk = (np.nonzero(valid)[0] + kph) // kv_block_size
             Mkv = (kph + N + kv_padding[1]) // kv_block_size
+            wg = 256 if D <= 160 else 128
             r = rs
             while r < re:  # rows of one workgroup share its parts
-                p0 = ((r + ph) // 256) * 256
-                r1 = min(re, p0 + 256 - ph)
-                part = _split_parts(merged_indices[b, h], q_block_size, N, ph, Mkv, splits, p0)
+                p0 = ((r + ph) // wg) * wg
+                r1 = min(re, p0 + wg - ph)
+                part = _split_parts(merged_indices[b, h], q_block_size, N, ph, Mkv, splits, p0, wg)
                 tp = np.array([part.get(int(m), -1) for m in tok_blk])
                 rows = r1 - r
                 acc = np.zeros((rows, D))

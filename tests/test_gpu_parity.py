@@ -435,6 +435,9 @@ def check_attn_vs_oracle(q, k, v, do, o, lse, merged, H, g, b, qpad, kvpad, dt, 
         vn = vn.reshape(B, N, -1, Dk).repeat(gqa_repeat, axis=2).reshape(B, N, C)
     # the forward ran through the Python API (with its workspace): small grids split the walks
     splits = _lib.lib().fta_sparse_attn_fwd_splits(B, H, N, C // H, g, b, qpad[0], qpad[1], kvpad[0], kvpad[1])
+    listed = min((N + sum(kvpad)) // b, -(-128 // g) * merged.shape[3]) * -(-b // 64)  # chunks of a walk, at most
+    if C // H > 160 and listed <= (6 if splits == 2 else 4):
+        splits = 1  # lists too short to split
     rr, rl = O.sparse_attn(qn, kn, vn, merged, H, g, b, None, qpad, kvpad, round_p=rk, splits=splits)
     assert_within(np32(o), rr, name="o vs rounding oracle")
     ro, _ = O.sparse_attn(qn, kn, vn, merged, H, g, b, None, qpad, kvpad)

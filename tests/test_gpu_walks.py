@@ -229,6 +229,33 @@ def test_wide_query_blocks(N, H, D, g):
         assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("H,g,b,W,short", [
+    (3, 64, 64, 2, True), (3, 32, 64, 1, True), (3, 64, 128, 1, True), (3, 33, 64, 1, True), (3, 64, 64, 3, False),
+    (3, 32, 64, 2, False), (12, 64, 64, 3, True), (12, 32, 64, 2, False)])  # 4 parts with 3 heads, 2 with 12
+def test_wide_head_short_lists(H, g, b, W, short):
+    """At D = 256 a small grid splits only walks of more than 4 chunks (6 in two parts):
+    shorter ones give the bits of the call without a workspace (unsplit)."""
+    from flash_topk_attn_v2 import _lib
+
+    N, D = 1056, 256
+    say(f"[short wide] H{H} g{g} b{b} W{W}")
+    qpad, kvpad = -N % g, -N % b
+    QM, M = (N + qpad) // g, (N + kvpad) // b
+    merged = torch.from_numpy(_random_merged(1, H, QM, W, M, 29)).cuda()
+    q, k, v = (rand((1, N, H * D), 84 + i, torch.bfloat16, "cuda") for i in range(3))
+    L, st = _lib.lib(), _lib.i64arr((N * H * D, D, H * D))
+    assert L.fta_sparse_attn_fwd_splits(1, H, N, D, g, b, 0, qpad, 0, kvpad) > 1
+    o, lse = fta.flash_topk_attn(q, k, v, merged, None, H, g, b, None, None, (0, kvpad), (0, qpad))
+    o2, lse2 = torch.empty_like(o), torch.empty_like(lse)
+    _lib.check(L.fta_sparse_attn_fwd_gqa(q.data_ptr(), st, k.data_ptr(), st, v.data_ptr(), st, 0, 1, H, H, N, D,
+                                         merged.data_ptr(), QM, W, g, b, 0, qpad, 0, kvpad, D ** -0.5, o2.data_ptr(), st,
+                                         lse2.data_ptr(), None, 0, torch.cuda.current_stream().cuda_stream), "fwd")
+    torch.cuda.synchronize()
+    assert torch.equal(o, o2) == short
+    if short:
+        assert torch.equal(lse, lse2)
+
+
 def _check_grads(tokens, lists, got, H, Hk, D, g, b):
     """dq, dk, dv (``got``) of one unpadded sequence against float64.  P and dS are rounded
     to 16 bits once (relative error u = 2^-9 or 2^-12) and so are o, which delta is formed
