@@ -251,8 +251,8 @@ size_t fta_sparse_attn_fwd_workspace_size(int B, int H, int N, int D, int q_bloc
  * each workgroup's walk over the union of its q-blocks' lists (ascending, per
  * 512-block segment) is split into that many contiguous ranges, each with its
  * own online-softmax anchor, and a combine kernel merges the parts' (O, max,
- * sum).  No counterpart in the reference (its forward is never split); exposed so that callers and tests can tell
- * which schedule rounds P.
+ * sum).  No counterpart in the reference (its forward is never split); exposed
+ * so that callers and tests can tell which schedule rounds P.
  */
 int fta_sparse_attn_fwd_splits(int B, int H, int N, int D, int q_block_size, int kv_block_size,
                                int q_pad_head, int q_pad_tail, int kv_pad_head, int kv_pad_tail);
